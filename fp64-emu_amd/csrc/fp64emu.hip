@@ -22,9 +22,11 @@
 //                  products run back to back; the epilogue reduces residue
 //                  slots to balanced int8 and stores correction slots as
 //                  raw int32.
-//   4. reconstruct reconstruct_kernel: balanced Garner digits with
-//                  v_dot4_i32_i8, grouped Horner, exact 128-bit combine with
-//                  the correction, correctly rounded conversion, rescale.
+//   4. reconstruct reconstruct_kernel: the exact combine of the usual plans
+//                  by remainder weights in three exact float64 slices (crt4),
+//                  otherwise balanced Garner digits with v_dot4_i32_i8 and
+//                  grouped Horner; the correction joins exactly, one
+//                  rounding, rescale.
 //
 // The arithmetic each stage computes follows fp64_emu_cuda/fp64_emu.cu of the
 // reference (line citations at each kernel); the data layouts, launch shapes
@@ -2429,7 +2431,10 @@ modgemm_split_x_kernel(GemmArgs g) {
 }
 
 // ---------------------------------------------------------------------------
-// Reconstruction.  Per output element: balanced Garner digits
+// Reconstruction.  Per output element, X from its residues, the correction
+// (corr1 + corr2) 2^(be - 15), one rounding to double, ldexp by -(sftA + sftB).
+// The exact combine of 12 to 15 default moduli sums remainder weights in
+// float64 (crt4); every other call takes balanced Garner digits
 //   d_t = bal((r_t - sum_{u<t} d_u (M_u mod p_t)) (M_t mod p_t)^-1 mod p_t)
 // with the O(P^2) inner products as v_dot4_i32_i8 over packed digits; Horner
 // per group of 7 moduli (the first four steps of a group in int32: a balanced
@@ -2550,6 +2555,279 @@ __device__ __forceinline__ double i128_to_f64(int64_t hi, uint64_t lo, int sh64)
   return ldexp(i64_to_f64((int64_t)top), sh64 - k);
 }
 
+// The default list's Chinese remainder weights, for the exact combine: with
+// W_t = (M / p_t) ((M / p_t)^-1 mod p_t) taken mod M in (-M/2, M/2], the
+// product is X = sum_t r_t W_t - q M for any residues r_t, q the nearest
+// integer to the sum over M.  W_t and M are cut into three slices of kCrtBits
+// bits (balanced, but for the top one), so that each slice's sum over
+// residues (or sums of a K-split's residues: crt_exact) is an exact float64
+// integer:  sum_t r_t W_t = s1 4^kCrtBits + s2 2^kCrtBits + s3.
+// The digits' serial chain, their 14-step Horner and the 128-bit combine took
+// 190 vector instructions an element at 14 moduli, this 120 with no serial
+// part, and a K-split's sums need no reduction first.  Whole calls against the
+// digits: 128 x 128 x 4096 (8 splits) 43.2 -> 41.3 us, 64 x 512^3 487.6 ->
+// 482.3 us, 1024^3 62.0 -> 60.6 us; from 4096^3 on even (the reconstruction
+// there streams 18 bytes in and 8 out an element at 5.5 TB/s either way).
+constexpr int kCrtBits = 39;
+
+struct CrtTab {
+  double w[3][kMaxP];   // slices of W_t, the top one first
+  double m[3];          // slices of M
+  double inv;           // 2^kCrtBits / M
+  double top;           // the largest |s| of any slice, before and after q M, at |r_t| <= p_t / 2
+};
+
+__host__ __device__ constexpr void crt_slices(i128 v, double (&out)[3]) {
+  for (int i = 2; i >= 1; --i) {
+    const i128 half = (i128)1 << (kCrtBits - 1);
+    const i128 low = ((v + half) & (((i128)1 << kCrtBits) - 1)) - half;
+    out[i] = (double)(long long)low;
+    v = (v - low) >> kCrtBits;
+  }
+  out[0] = (double)(long long)v;
+}
+
+__host__ __device__ constexpr CrtTab crt_tables(int P) {
+  CrtTab T{};
+  i128 M = 1;
+  for (int t = 0; t < P; ++t) M *= kDefaultModuli[t];
+  double sums[3] = {0.0, 0.0, 0.0}, all = 0.0;
+  for (int t = 0; t < P; ++t) {
+    const int p = kDefaultModuli[t];
+    const i128 N = M / p;
+    i128 W = N * inv_mod((int)(N % p), p);
+    if (2 * W > M) W -= M;
+    double s[3] = {};
+    crt_slices(W, s);
+    for (int i = 0; i < 3; ++i) {
+      T.w[i][t] = s[i];
+      sums[i] += (double)(p / 2) * (s[i] < 0 ? -s[i] : s[i]);
+    }
+    all += (double)(p / 2) * (double)(W < 0 ? -W : W);
+  }
+  crt_slices(M, T.m);
+  T.inv = (double)(1ll << kCrtBits) / (double)M;
+  for (int i = 0; i < 3; ++i) {
+    const double v = sums[i] + (all / (double)M + 1.0) * (T.m[i] < 0 ? -T.m[i] : T.m[i]);
+    T.top = v > T.top ? v : T.top;
+  }
+  return T;
+}
+
+// Modulus counts whose sums of residues |r_t| <= 128 fold stay exact.
+__host__ __device__ constexpr bool crt_exact(int P, int fold) {
+  if (P < 12 || P > 15) return false;
+  return crt_tables(P).top * fold < 9007199254740992.0;   // 2^53
+}
+
+// RN(X + cv 2^cshift) 2^sh for the slice sums s1, s2, s3 of an element (before
+// the multiple of M comes off): exactly rounded, as the 128-bit combine.  Every
+// value is an integer, and each Fast2Sum's first operand a multiple of the
+// second one's ulp (a slice of weight 2^39 against at most 52 bits below 2^91,
+// and so on), which makes its error exact whichever operand is larger.
+template <int kP>
+__host__ __device__ __forceinline__ double crt_combine(double s1, double s2, double s3, const double cv,
+                                                       const int cshift, const int sh) {
+  constexpr CrtTab T = crt_tables(kP);
+  constexpr double kB = (double)(1ll << kCrtBits);
+  // The nearest integer to the sum over M, from the sum's top 53 bits: off
+  // only within 2^-40 of a tie, while the width pick keeps |X| below 0.36 M.
+  const double q = fma(fma(s1, kB, s2), T.inv, kMagic) - kMagic;
+  s1 = fma(-q, T.m[0], s1);
+  s2 = fma(-q, T.m[1], s2);
+  s3 = fma(-q, T.m[2], s3);
+  // (h, l) = s1 2^39 + s2, in units of 2^39.
+  const double h = fma(s1, kB, s2);
+  const double l = s2 - fma(s1, -kB, h);
+  // (u, v) = the correction + s3.
+  const double d = ldexp(cv, cshift);
+  const double u = d + s3;
+  const double v = s3 - (u - d);
+  // (p, e) = l + u, (h2, p2) = h + p: the value is h2 + p2 + (e + v).
+  const double p = fma(l, kB, u);
+  const double e = u - fma(l, -kB, p);
+  const double h2 = fma(h, kB, p);
+  const double p2 = p - fma(h, -kB, h2);
+  // p2 + (e + v) rounded to odd (its last bit set when inexact), so that the
+  // last addition rounds once: it is inexact only beyond 2^53, when h2 is
+  // beyond 2^105 and its rounding position far above that bit.
+  const double s = e + v;
+  const double y = p2 + s;
+  const double err = s - (y - p2);
+  uint64_t yb;
+  __builtin_memcpy(&yb, &y, 8);
+  uint64_t eb;
+  __builtin_memcpy(&eb, &err, 8);
+  const bool inexact = err != 0.0;
+  const int64_t opposite = (int64_t)(eb ^ yb) >> 63;   // -1: |y| is above the exact magnitude
+  yb = inexact ? (yb + (uint64_t)opposite) | 1u : yb;
+  double yo;
+  __builtin_memcpy(&yo, &yb, 8);
+  return ldexp(h2 + yo, sh);
+}
+
+// Four elements' values from their residues r(t, e) (any representatives, or
+// sums of representatives: crt_exact), correction sums cv and shifts.
+template <int kP, typename R>
+__device__ __forceinline__ void crt4(const R& r, const double (&cv)[4], const int cshift,
+                                     const int (&sh)[4], double (&val)[4]) {
+  constexpr CrtTab T = crt_tables(kP);
+  double s1[4] = {0.0, 0.0, 0.0, 0.0}, s2[4] = {0.0, 0.0, 0.0, 0.0}, s3[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int t = 0; t < kP; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const double d = (double)r(t, e);
+      s1[e] = fma(d, T.w[0][t], s1[e]);
+      s2[e] = fma(d, T.w[1][t], s2[e]);
+      s3[e] = fma(d, T.w[2][t], s3[e]);
+    }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) val[e] = crt_combine<kP>(s1[e], s2[e], s3[e], cv[e], cshift, sh[e]);
+}
+
+// One element's value from its Horner group values a0, a1, a2 (ng of them
+// used), the group products m0, m1 and the correction sum cv, scaled by 2^sh.
+// short_top: a1 + m1 a2 fits 63 bits.
+template <bool kExact>
+__device__ __forceinline__ double combine_groups(const long long a0, const long long a1, const long long a2,
+                                                 const int ng, const bool short_top, const long long m0,
+                                                 const long long m1, const int64_t cv, const int cshift,
+                                                 const int sh) {
+  if constexpr (kExact) {
+    // X = a0 + M0 (a1 + M1 a2) as a 128-bit word pair (hi, lo).  The one
+    // or two group products of the usual plans (at most 15 moduli: group 2
+    // holds at most one digit, so a1 + M1 a2 fits 63 bits) take
+    // mul_add_wide's four 32 x 32 -> 64 multiply-adds; longer lists take
+    // the general 128-bit product (the true X stays below 2^127, so the
+    // products wrap modulo 2^128 harmlessly).
+    uint64_t lo;
+    int64_t hi;
+    if (ng == 1) {
+      lo = (uint64_t)a0;
+      hi = a0 >> 63;
+    } else if (ng == 2 || short_top) {
+      const int64_t top = ng == 2 ? a1 : (int64_t)((uint64_t)a2 * (uint64_t)m1) + a1;
+      mul_add_wide(top, (uint64_t)m0, a0, lo, hi);
+    } else {
+      i128 acc = (i128)a2 * (i128)(uint64_t)m1 + a1;
+      acc = acc * (i128)(uint64_t)m0 + a0;
+      lo = (uint64_t)acc;
+      hi = (int64_t)(acc >> 64);
+    }
+    // + corr 2^cshift: 1 <= cshift <= 38 (bits_eff in [16, 53]), so the
+    // shifted value is the word pair (cv >> (64 - cshift), cv << cshift).
+    const unsigned __int128 cw =
+        ((unsigned __int128)(uint64_t)(cv >> (64 - cshift)) << 64) | ((uint64_t)cv << cshift);
+    const unsigned __int128 u = (((unsigned __int128)(uint64_t)hi << 64) | lo) + cw;
+    return i128_to_f64((int64_t)(u >> 64), (uint64_t)u, 64 + sh);
+  } else {
+    double acc = (double)(ng == 3 ? a2 : (ng == 2 ? a1 : a0));
+    if (ng == 3) acc = fma(acc, (double)m1, (double)a1);
+    if (ng >= 2) acc = fma(acc, (double)m0, (double)a0);
+    acc = acc + ldexp((double)cv, cshift);
+    return ldexp(acc, sh);
+  }
+}
+
+// Four elements (the bytes of the residue words w[0 .. kP)) of a product over
+// the default modulus list: Garner digits, Horner and the exact or float64
+// combine with the correction sums cv, scaled by 2^sh[e].
+template <bool kExact, int kP>
+__device__ __forceinline__ void reconstruct4(const uint32_t (&w)[kMaxP], const int64_t (&cv)[4],
+                                             const int cshift, const int (&sh)[4], double (&val)[4]) {
+  // The digits of X + M/2, in [0, p_t) (default_digit_offset): digit 0 is
+  // r_0 + 128, the residue byte with its top bit flipped; digit t is y mod
+  // p_t for y = 128 p_t + r_t minv_t + sum_{u<t} d_u (-M_u minv_t mod p_t),
+  // the sum as unsigned dot products of digit bytes and factor bytes in
+  // [0, p_t), so 0 < y < 2^21 and its quotient by p_t is one high multiply
+  // (mq = ceil(2^32 / p_t): exact below 2^24).
+  int dg[4][kMaxP];
+  int dp[4][kGarnerWords];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int g = 0; g < kGarnerWords; ++g) dp[e][g] = 0;
+  const uint32_t u0 = w[0] ^ 0x80808080u;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t s0 = u0 >> (8 * e);
+    dg[e][0] = (int)(s0 & 0xFFu);
+    dp[e][0] = (int)s0;   // bytes 1..3 meet zero factors until digits 1..3 land there
+  }
+#pragma unroll
+  for (int t = 1; t < kP; ++t) {
+    const int pt = kDefaultModuli[t];
+    const int mib = kDefaultTab.mib[t];
+    const uint32_t mq = kDefaultTab.mq[t];
+    const int bsh = 8 * (t & 3);
+    // 128 p_t in one register for the four elements' first dot products
+    // (kept opaque: the compiler would otherwise rematerialise it into each
+    // chain's accumulator, one move per element).
+    uint32_t bias;
+    asm volatile("v_mov_b32 %0, %1" : "=v"(bias) : "i"(128 * pt));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      // The digits' terms first (from 128 p_t), then r_t minv_t from byte e
+      // of the residue word (the factor word holds minv_t at byte e only).
+      // (Issuing the residue term first, off the digit-to-digit chain, in
+      // the three-operand form with the factor in a scalar register
+      // measured 3% slower at 8192^3.)
+      uint32_t y = bias;
+#pragma unroll
+      for (int g = 0; g < kGarnerWords; ++g)
+        if (4 * g < t)
+          y = __builtin_amdgcn_udot4((uint32_t)dp[e][g], kDefaultTab.ump[t * kGarnerWords + g], y, false);
+      y = (uint32_t)__builtin_amdgcn_sdot4((int)w[t], (int)((uint32_t)(uint8_t)(int8_t)mib << (8 * e)),
+                                           (int)y, false);
+      const int d = __mul24((int)__umulhi(y, mq), -pt) + (int)y;
+      dg[e][t] = d;
+      dp[e][t >> 2] = (t & 3) == 0 ? d
+                                   : (int)__builtin_amdgcn_perm((uint32_t)d, (uint32_t)dp[e][t >> 2],
+                                                                 (0x03020100u & ~(0xFFu << bsh)) | (0x04u << bsh));
+    }
+  }
+
+  // Horner per group of 7 (digits 7g .. 7g+6, high to low), in two 32-bit
+  // halves: positions 6..3 give H (below p_3 p_4 p_5 p_6 < 2^32), positions
+  // 2..0 give L (below 2^24), and the group value is H (p_0 p_1 p_2) + L, one
+  // 32 x 32 -> 64-bit multiply-add (p_i the group's first three moduli; a
+  // group of at most three digits has H = 0), less the group's digit offset.
+  // Every partial H below its last step is below 2^24, so the 24-bit
+  // multiplies are exact.
+  long long ag[4][3];
+  uint32_t h32[4][3], l32[4][3];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int g = 0; g < 3; ++g) { h32[e][g] = 0u; l32[e][g] = 0u; }
+#pragma unroll
+  for (int t = kP - 1; t >= 0; --t) {
+    const int g = t / 7, pos = t % 7;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (pos >= 3) h32[e][g] = __umul24(h32[e][g], (uint32_t)kDefaultModuli[t]) + (uint32_t)dg[e][t];
+      else l32[e][g] = __umul24(l32[e][g], (uint32_t)kDefaultModuli[t]) + (uint32_t)dg[e][t];
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 3; ++g) {
+    const int t0 = 7 * g;
+    const uint32_t p3 = t0 + 2 < kMaxP ? (uint32_t)(kDefaultModuli[t0] * kDefaultModuli[t0 + 1] *
+                                                    kDefaultModuli[t0 + 2]) : 0u;
+    const long long off = default_digit_offset(kP, g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      ag[e][g] = (long long)((unsigned long long)h32[e][g] * p3 + l32[e][g]) - off;
+  }
+
+  constexpr int ng = (kP + 6) / 7;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    val[e] = combine_groups<kExact>(ag[e][0], ag[e][1], ag[e][2], ng, kP == 15 || ng < 3, kDefaultM64[0],
+                                    kDefaultM64[1], cv[e], cshift, sh[e]);
+}
+
 struct ReconCore {
   const int8_t* res8;
   const int32_t* corr;
@@ -2603,6 +2881,8 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
 
   const int P = kP > 0 ? kP : a.P;
   constexpr bool kUsual = kP > 0;
+  // Exact combine of the usual plans: by remainder weights, not Garner digits.
+  constexpr bool kCrt = kUsual && kExact && crt_exact(kP, 1);
   // Table entries: compile-time constants of the default modulus list in
   // the specialised kernels (no scalar registers held across the kernel and
   // no tables among the arguments), kernel arguments otherwise.
@@ -2637,8 +2917,19 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
   int sai[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) sai[e] = (int)load_at<int16_t>(sftA_blk, 2u * min(row0 + e, last_row));
+  // The wave's output rows from a uniform base; the lane's byte offset is
+  // its column's.
+  double* const oblk = a.out + ((int64_t)b * a.M + (int64_t)mb * 16 + row0) * a.N + (int64_t)nb * 64;
+  const uint32_t olane = 8u * (uint32_t)col;
+  auto store4 = [&](const double (&val)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (row0 + e < rows_left) store_at<double>(oblk + e * a.N, olane, val[e]);
+  };
   uint32_t w[kMaxP];
-  int64_t cv[4] = {0, 0, 0, 0};
+  // The correction sums, exact either way.
+  typedef std::conditional_t<kCrt, double, int64_t> CorrSum;
+  CorrSum cv[4] = {0, 0, 0, 0};
   if (kDeep) {
     // Fold the segment sums (|sum| <= 128 per segment and split) to balanced
     // residues; the S splits' sums add first, and so do their correction
@@ -2709,8 +3000,20 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
         for (int cc = 0; cc < 2; ++cc)
           if (cc < a.ncorr) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) cv[e] += cw[h][cc][e];
+            for (int e = 0; e < 4; ++e) cv[e] += (CorrSum)cw[h][cc][e];
           }
+      }
+    }
+    if constexpr (kCrt) {
+      if (crt_exact(kP, kMaxSplit) || a.ksplit * 2 <= kMaxSplit) {
+        static_assert(crt_exact(kP, kMaxSplit / 2), "remainder weights: sums of half the largest K-split");
+        int sh[4];
+        double val[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sh[e] = -(sai[e] + sj);
+        crt4<kP>([&](int t, int e) { return sums[t][e]; }, cv, cshift, sh, val);
+        store4(val);
+        return;
       }
     }
 #pragma unroll
@@ -2731,14 +3034,28 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
     const int32_t* cb = a.corr + (int64_t)b * a.ncorr * a.outplane + boff0;
     const v4i c1 = load_at<v4i>(cb, 4 * lane4);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) cv[e] = c1[e];
+    for (int e = 0; e < 4; ++e) cv[e] = (CorrSum)c1[e];
     if (a.ncorr == 2) {
       const v4i c2 = load_at<v4i>(cb + a.outplane, 4 * lane4);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) cv[e] += c2[e];
+      for (int e = 0; e < 4; ++e) cv[e] += (CorrSum)c2[e];
     }
   }
 
+
+  if constexpr (kUsual) {
+    int sh[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sh[e] = -(sai[e] + sj);
+    double val[4];
+    if constexpr (kCrt) {
+      crt4<kP>([&](int t, int e) { return (int)(int8_t)(uint8_t)(w[t] >> (8 * e)); }, cv, cshift, sh, val);
+    } else {
+      reconstruct4<kExact, kP>(w, cv, cshift, sh, val);
+    }
+    store4(val);
+    return;
+  }
 
   // Garner digits, 4 elements in lockstep.
   int dg[4][kMaxP];
@@ -2747,54 +3064,7 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
   for (int e = 0; e < 4; ++e)
 #pragma unroll
     for (int g = 0; g < kGarnerWords; ++g) dp[e][g] = 0;
-  if constexpr (kUsual) {
-    // The digits of X + M/2, in [0, p_t) (default_digit_offset): digit 0 is
-    // r_0 + 128, the residue byte with its top bit flipped; digit t is y mod
-    // p_t for y = 128 p_t + r_t minv_t + sum_{u<t} d_u (-M_u minv_t mod p_t),
-    // the sum as unsigned dot products of digit bytes and factor bytes in
-    // [0, p_t), so 0 < y < 2^21 and its quotient by p_t is one high multiply
-    // (mq = ceil(2^32 / p_t): exact below 2^24).
-    const uint32_t u0 = w[0] ^ 0x80808080u;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t s0 = u0 >> (8 * e);
-      dg[e][0] = (int)(s0 & 0xFFu);
-      dp[e][0] = (int)s0;   // bytes 1..3 meet zero factors until digits 1..3 land there
-    }
-#pragma unroll
-    for (int t = 1; t < kMaxP; ++t) {
-      if (t >= P) continue;
-      const int pt = kDefaultModuli[t];
-      const int mib = kDefaultTab.mib[t];
-      const uint32_t mq = kDefaultTab.mq[t];
-      const int sh = 8 * (t & 3);
-      // 128 p_t in one register for the four elements' first dot products
-      // (kept opaque: the compiler would otherwise rematerialise it into each
-      // chain's accumulator, one move per element).
-      uint32_t bias;
-      asm volatile("v_mov_b32 %0, %1" : "=v"(bias) : "i"(128 * pt));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        // The digits' terms first (from 128 p_t), then r_t minv_t from byte e
-        // of the residue word (the factor word holds minv_t at byte e only).
-        // (Issuing the residue term first, off the digit-to-digit chain, in
-        // the three-operand form with the factor in a scalar register
-        // measured 3% slower at 8192^3.)
-        uint32_t y = bias;
-#pragma unroll
-        for (int g = 0; g < kGarnerWords; ++g)
-          if (4 * g < t)
-            y = __builtin_amdgcn_udot4((uint32_t)dp[e][g], kDefaultTab.ump[t * kGarnerWords + g], y, false);
-        y = (uint32_t)__builtin_amdgcn_sdot4((int)w[t], (int)((uint32_t)(uint8_t)(int8_t)mib << (8 * e)),
-                                             (int)y, false);
-        const int d = __mul24((int)__umulhi(y, mq), -pt) + (int)y;
-        dg[e][t] = d;
-        dp[e][t >> 2] = (t & 3) == 0 ? d
-                                     : (int)__builtin_amdgcn_perm((uint32_t)d, (uint32_t)dp[e][t >> 2],
-                                                                   (0x03020100u & ~(0xFFu << sh)) | (0x04u << sh));
-      }
-    }
-  } else {
+  {
 #pragma unroll
     for (int t = 0; t < kMaxP; ++t) {
       if (t >= P) continue;
@@ -2847,47 +3117,14 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
     }
   }
 
-  // The wave's output rows from a uniform base; the lane's byte offset is
-  // its column's.
-  double* const oblk = a.out + ((int64_t)b * a.M + (int64_t)mb * 16 + row0) * a.N + (int64_t)nb * 64;
-  const uint32_t olane = 8u * (uint32_t)col;
-
   // Horner per group of 7 (digits 7g .. 7g+6, high to low), in two 32-bit
   // halves: positions 6..3 give H, positions 2..0 give L (below 2^24), and
   // the group value is H (p_0 p_1 p_2) + L, one 32 x 32 -> 64-bit
   // multiply-add (p_i the group's first three moduli; a group of at most
   // three digits has H = 0).  Every partial H below its last step is below
   // 2^24, so the 24-bit multiplies are exact.  Balanced digits: |H| < 2^31.
-  // Default-list digits (in [0, p)): H < p_3 p_4 p_5 p_6 < 2^32 unsigned, and
-  // the group's digit offset comes off the 64-bit value.
   long long ag[4][3];
-  if constexpr (kUsual) {
-    uint32_t h32[4][3], l32[4][3];
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int g = 0; g < 3; ++g) { h32[e][g] = 0u; l32[e][g] = 0u; }
-#pragma unroll
-    for (int t = kMaxP - 1; t >= 0; --t) {
-      if (t >= P) continue;
-      const int g = t / 7, pos = t % 7;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (pos >= 3) h32[e][g] = __umul24(h32[e][g], (uint32_t)kDefaultModuli[t]) + (uint32_t)dg[e][t];
-        else l32[e][g] = __umul24(l32[e][g], (uint32_t)kDefaultModuli[t]) + (uint32_t)dg[e][t];
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < 3; ++g) {
-      const int t0 = 7 * g;
-      const uint32_t p3 = t0 + 2 < kMaxP ? (uint32_t)(kDefaultModuli[t0] * kDefaultModuli[t0 + 1] *
-                                                      kDefaultModuli[t0 + 2]) : 0u;
-      const long long off = default_digit_offset(kP, g);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        ag[e][g] = (long long)((unsigned long long)h32[e][g] * p3 + l32[e][g]) - off;
-    }
-  } else {
+  {
     int h32[4][3], l32[4][3];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -2919,47 +3156,9 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
     if (row0 + e >= rows_left) continue;
     // Every group ends on its position-0 digit, an int64 step, so ag holds
     // the group value whatever the group's digit count.
-    const long long a0 = ag[e][0], a1 = ag[e][1], a2 = ag[e][2];
-    const int sh = -(sai[e] + sj);
-    double val;
-    if (kExact) {
-      // X = a0 + M0 (a1 + M1 a2) as a 128-bit word pair (hi, lo).  The one
-      // or two group products of the usual plans (at most 15 moduli: group 2
-      // holds at most one digit, so a1 + M1 a2 fits 63 bits) take
-      // mul_add_wide's four 32 x 32 -> 64 multiply-adds; longer lists take
-      // the general 128-bit product (the true X stays below 2^127, so the
-      // products wrap modulo 2^128 harmlessly).
-      const uint64_t m0 = (uint64_t)tab_m64(0);
-      const uint64_t m1 = (uint64_t)tab_m64(1);
-      uint64_t lo;
-      int64_t hi;
-      if (ng == 1) {
-        lo = (uint64_t)a0;
-        hi = a0 >> 63;
-      } else if (ng == 2 || (kUsual && P == 15)) {
-        const int64_t top = ng == 2 ? a1 : (int64_t)((uint64_t)a2 * m1) + a1;
-        mul_add_wide(top, m0, a0, lo, hi);
-      } else {
-        i128 acc = (i128)a2 * (i128)m1 + a1;
-        acc = acc * (i128)m0 + a0;
-        lo = (uint64_t)acc;
-        hi = (int64_t)(acc >> 64);
-      }
-      // + corr 2^cshift: 1 <= cshift <= 38 (bits_eff in [16, 53]), so the
-      // shifted value is the word pair (cv >> (64 - cshift), cv << cshift).
-      const unsigned __int128 cw =
-          ((unsigned __int128)(uint64_t)(cv[e] >> (64 - cshift)) << 64) | ((uint64_t)cv[e] << cshift);
-      const unsigned __int128 u = (((unsigned __int128)(uint64_t)hi << 64) | lo) + cw;
-      store_at<double>(oblk + e * a.N, olane, i128_to_f64((int64_t)(u >> 64), (uint64_t)u, 64 + sh));
-      continue;
-    } else {
-      double acc = (double)(ng == 3 ? a2 : (ng == 2 ? a1 : a0));
-      if (ng == 3) acc = fma(acc, (double)tab_m64(1), (double)a1);
-      if (ng >= 2) acc = fma(acc, (double)tab_m64(0), (double)a0);
-      acc = acc + ldexp((double)cv[e], cshift);
-      val = acc;
-    }
-    store_at<double>(oblk + e * a.N, olane, ldexp(val, sh));
+    store_at<double>(oblk + e * a.N, olane,
+                     combine_groups<kExact>(ag[e][0], ag[e][1], ag[e][2], ng, false, tab_m64(0), tab_m64(1),
+                                            (int64_t)cv[e], cshift, -(sai[e] + sj)));
   }
 }
 
