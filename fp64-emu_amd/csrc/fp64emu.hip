@@ -423,17 +423,42 @@ bool use_split_streams(const fp64emu_layout_t& L) {
   return (units + 31) / 32 >= 8;
 }
 
+// Whole-K products (K > 131071, fp64emu_product): planes over the whole depth
+// and one launch of K-split groups, each below the int32 bound, instead of
+// one extraction and one accumulating GEMM per segment.  The K-split fills
+// the chip's group slots (kGroupsPerCU per CU) in as few rounds as the work
+// allows: of the counts up to kMaxSplit, the one with the least
+// rounds x k-steps a group, plus the split planes' traffic.  Against the
+// segments (each an extraction writing the padded rows too, then a GEMM of
+// 256 x 256 tiles reading and writing int32 sums of every split): 300 x 200 x
+// 200000 1873 -> 1207 us, its GEMM 1074 -> 540 us (2.0 GB of planes once, at
+// 3.6 TB/s) and its extraction 613 -> 538 us (2.8 GB at 5.1 TB/s).
+int choose_whole_k_split(int64_t items, int64_t nkt, int64_t group_slots, double step_seconds,
+                         double split_seconds) {
+  int best = kMaxSplit;
+  double best_t = 1e300;
+  for (int S = (int)((nkt + kMaxKSingle / kTileK - 1) / (kMaxKSingle / kTileK)); S <= kMaxSplit; ++S) {
+    const int64_t rounds = (items * S + group_slots - 1) / group_slots;
+    const double t = (double)rounds * ((double)((nkt + S - 1) / S) + 6.0) * step_seconds + S * split_seconds;
+    if (t < best_t) { best_t = t; best = S; }
+  }
+  return best;
+}
+
+bool whole_k_possible(int64_t K) { return K > kMaxKSingle && K <= kMaxSplit * (kMaxKSingle / kTileK * kTileK); }
+
 // nchunk_req > 1 (batch 1, not K-segmented): the planes of A and the output
 // planes hold one chunk of ceil(TM / nchunk_req) row tiles at a time.
+// whole_k: the whole-K form of a product deeper than one launch's bound.
 void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool corr,
-                 fp64emu_layout_t* L, int64_t nchunk_req = 1) {
+                 fp64emu_layout_t* L, int64_t nchunk_req = 1, bool whole_k = false) {
   std::memset(L, 0, sizeof(*L));
   L->batch = batch; L->M = M; L->N = N; L->K = K;
   L->nprimes = P; L->use_corr = corr ? 1 : 0;
   // K-segmented (K > 131071, B as [N, K]): planes hold one segment; each
   // segment's correction is one fused GEMM; the GEMMs accumulate into int32
   // residue sums and one int64 correction sum.
-  L->deep = K > kMaxKSingle ? 1 : 0;
+  L->deep = K > kMaxKSingle && !whole_k ? 1 : 0;
   L->kseg = L->deep ? kSegK : K;
   L->nseg = L->deep ? (int)((K + kSegK - 1) / kSegK) : 1;
   L->ncorr = corr ? ((L->deep || K <= kMaxKFusedCorr) ? 1 : 2) : 0;
@@ -458,11 +483,23 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
   // and int64 correction sums across the segments.)
   L->ksplit = choose_ksplit(batch, ctiles * (L->Np / kTileR), L->Kp / kTileK, P, L->ncorr,
                             batch * L->outplane_bytes, batch * (L->memberA_bytes + L->memberB_bytes));
+  bool whole_k_small = false;
+  if (whole_k) {
+    // 128 x 128 tiles (two groups per CU) where they cut the padded work by
+    // more than 10%.
+    const int64_t rows128 = round_up(std::max<int64_t>(M, 1), 128), cols128 = round_up(std::max<int64_t>(N, 1), 128);
+    whole_k_small = rows128 * cols128 * 11 < L->Mp * L->Np * 10;
+    const int64_t tiles = whole_k_small ? rows128 / 128 * (cols128 / 128) : TM * (L->Np / kTileR);
+    const int slots = P + (corr ? 2 : 0);
+    L->ksplit = choose_whole_k_split(batch * tiles * slots, L->Kp / kTileK, whole_k_small ? 2 * kCUs : kCUs,
+                                     whole_k_small ? 0.37e-6 : 0.73e-6,
+                                     (double)(batch * L->outplane_bytes) * (P + (corr ? 8 : 0)) / 4.0e12);
+  }
   // Under a K-split the two correction products run as two K-deep slots
   // (two int32 planes): a fused 2K-deep slot would make its groups twice as
   // long as every residue group (choose_ksplit already counts it as two).
   if (L->ksplit > 1 && L->ncorr == 1) L->ncorr = 2;
-  if (use_split_streams(*L)) {
+  if (!whole_k && use_split_streams(*L)) {
     L->gemm_split = 1;
     L->ksplit = 2;
   }
@@ -505,6 +542,7 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
       if (L->nchunk == 1 && tiles <= 40) L->gemm_tile_rows = 128;
     }
   }
+  if (whole_k) L->gemm_tile_rows = L->gemm_tile_cols = whole_k_small ? 128 : 256;
   L->gemm_run = use_slot_runs(*L) ? slot_run_length(*L) : 1;
   // Plane rows the GEMM reads: 128-row (128-column) tiles read only the
   // first half of a 256-row plane tile past the last one holding data, so
@@ -516,6 +554,25 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
   else
     L->ext_rowsB = (L->gemm_tile_cols == 128 || use_mixed_tiles(*L))
                        ? round_up(std::max<int64_t>(N, 1), 128) : L->Np;
+}
+
+// The layout of fp64emu_product, which leaves no stage for inspection: rows
+// past the operands' last 64-row group are never written (a GEMM output
+// depends on its own row and column alone, and the reconstruction reads the
+// valid ones), and a product past one launch's depth runs whole (whole_k)
+// while its workspace stays below kWholeKBytes.
+constexpr size_t kWholeKBytes = (size_t)24 << 30;
+
+void make_product_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool corr,
+                         fp64emu_layout_t* L) {
+  bool whole = whole_k_possible(K);
+  make_layout(batch, M, N, K, P, corr, L, 1, whole);
+  if (whole && L->total > kWholeKBytes) {
+    whole = false;
+    make_layout(batch, M, N, K, P, corr, L);
+  }
+  L->ext_rowsA = round_up(std::max<int64_t>(M, 1), 64);
+  L->ext_rowsB = round_up(std::max<int64_t>(N, 1), 64);
 }
 
 // ---------------------------------------------------------------------------
@@ -3427,6 +3484,7 @@ struct Call {
   size_t ws_bytes;
   hipStream_t stream;
   hipEvent_t* ev;   // 5 events or nullptr
+  bool product;     // fp64emu_product: no stage is kept for inspection
 };
 
 int check_hip(hipError_t e, const char* what) {
@@ -3499,7 +3557,9 @@ int run(const Call& c) {
     return fail(FP64EMU_EINVAL, "K bound for int32 modular GEMM");
   if (c.K > kMaxKDeep) return fail(FP64EMU_EINVAL, "K bound: 128 segments of 65536");
   fp64emu_layout_t L;
-  make_layout(c.batch, c.M, c.N, c.K, c.P, c.corr, &L);
+  if (c.product) make_product_layout(c.batch, c.M, c.N, c.K, c.P, c.corr, &L);
+  // (A product on a shorter workspace runs as the other entry points do.)
+  if (!c.product || c.ws_bytes < L.total) make_layout(c.batch, c.M, c.N, c.K, c.P, c.corr, &L);
   const hipStream_t s = c.stream;
   if (c.ev) {
     if (int st = check_hip(hipEventRecord(c.ev[0], s), "hipEventRecord")) return st;
@@ -3802,6 +3862,7 @@ Call make_call(double* out, const double* A, const double* B, int64_t batch, int
   c.ws = ws; c.ws_bytes = ws_bytes;
   c.stream = reinterpret_cast<hipStream_t>(stream);
   c.ev = nullptr;
+  c.product = false;
   return c;
 }
 
@@ -3863,6 +3924,24 @@ size_t fp64emu_workspace_size_min(int64_t batch, int64_t M, int64_t N, int64_t K
   fp64emu_layout_t L;
   make_layout(batch, M, N, K, nprimes, use_corr != 0, &L, round_up(std::max<int64_t>(M, 1), kTileR) / kTileR);
   return L.total;
+}
+
+size_t fp64emu_product_workspace(const fp64emu_product_t* p) {
+  if (!p || p->batch < 0 || p->M < 0 || p->N < 0 || p->K < 0 || p->nprimes < 1 || p->nprimes > kMaxP)
+    return 0;
+  fp64emu_layout_t L;
+  make_product_layout(p->batch, p->M, p->N, p->K, p->nprimes, p->use_corr != 0, &L);
+  return L.total;
+}
+
+int fp64emu_product(const fp64emu_product_t* p, void* workspace, size_t workspace_bytes,
+                    fp64emu_stream_t stream) {
+  g_err.clear();
+  if (!p) return fail(FP64EMU_EINVAL, "product must not be NULL");
+  Call c = make_call(p->out, p->A, p->B, p->batch, p->M, p->N, p->K, p->b_kn != 0, p->primes,
+                     p->nprimes, p->exact, p->bits, p->use_corr, workspace, workspace_bytes, stream);
+  c.product = true;
+  return run(c);
 }
 
 int fp64emu_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int nprimes, int use_corr,

@@ -70,6 +70,28 @@ void check_out(const at::Tensor& out, const at::Tensor& A, at::IntArrayRef sizes
   TORCH_CHECK(out.device() == A.device(), "out must be on the device of A");
 }
 
+// The product of checked operands (A as [batch, M, K]) into out.
+void product(at::Tensor& out, const at::Tensor& A, const at::Tensor& B, int64_t batch, int64_t M,
+             int64_t N, int64_t K, bool b_kn, const at::Tensor& primes_cpu, bool exact, int64_t bits,
+             bool use_corr) {
+  const c10::DeviceGuard guard(A.device());
+  const std::vector<int32_t> pv = primes_vec(primes_cpu);
+  fp64emu_product_t p;
+  p.out = out.data_ptr<double>();
+  p.A = A.data_ptr<double>();
+  p.B = B.data_ptr<double>();
+  p.batch = batch; p.M = M; p.N = N; p.K = K;
+  p.b_kn = b_kn;
+  p.primes = pv.data();
+  p.nprimes = (int)pv.size();
+  p.exact = exact;
+  p.bits = bits;
+  p.use_corr = use_corr;
+  at::Tensor ws = workspace_fit(A, fp64emu_product_workspace(&p),
+                                fp64emu_workspace_size_min(batch, M, N, K, p.nprimes, use_corr));
+  check_status(fp64emu_product(&p, ws.data_ptr(), (size_t)ws.numel(), current_stream(A)));
+}
+
 }  // namespace
 
 int64_t fp64_emu_maxp() { return fp64emu_maxp(); }
@@ -86,14 +108,7 @@ void fp64_emu_mm(at::Tensor& out, const at::Tensor& A, const at::Tensor& B,
   check_out(out, A, {M, N}, "out f64 [M,N]");
   // Deeper than 131071 runs K-segmented, to 128 segments of 65536.
   TORCH_CHECK(K <= kMaxKDeep, "K bound: 128 segments of 65536");
-  const c10::DeviceGuard guard(A.device());
-  const std::vector<int32_t> pv = primes_vec(primes_cpu);
-  const int P = (int)pv.size();
-  at::Tensor ws = workspace_fit(A, fp64emu_workspace_size(1, M, N, K, P, use_corr),
-                                fp64emu_workspace_size_min(1, M, N, K, P, use_corr));
-  check_status(fp64emu_mm(out.data_ptr<double>(), A.data_ptr<double>(), B.data_ptr<double>(), M,
-                          N, K, pv.data(), nullptr, nullptr, P, exact, bits, use_corr,
-                          ws.data_ptr(), (size_t)ws.numel(), current_stream(A)));
+  product(out, A, B, 1, M, N, K, false, primes_cpu, exact, bits, use_corr);
 }
 
 // out[m,n] = A[m,k] @ Bt[k,n], Bt in its [K, N] layout.
@@ -109,14 +124,7 @@ void fp64_emu_mm_nt(at::Tensor& out, const at::Tensor& A, const at::Tensor& Bt,
   TORCH_CHECK(Bt.size(0) == K, "expect Bt as [K, N]");
   check_out(out, A, {M, N}, "out f64 [M,N]");
   TORCH_CHECK(K <= kMaxKSingle, "K bound for int32 modular GEMM");
-  const c10::DeviceGuard guard(A.device());
-  const std::vector<int32_t> pv = primes_vec(primes_cpu);
-  const int P = (int)pv.size();
-  at::Tensor ws = workspace_fit(A, fp64emu_workspace_size(1, M, N, K, P, use_corr),
-                                fp64emu_workspace_size_min(1, M, N, K, P, use_corr));
-  check_status(fp64emu_mm_nt(out.data_ptr<double>(), A.data_ptr<double>(), Bt.data_ptr<double>(),
-                             M, N, K, pv.data(), nullptr, nullptr, P, exact, bits, use_corr,
-                             ws.data_ptr(), (size_t)ws.numel(), current_stream(A)));
+  product(out, A, Bt, 1, M, N, K, true, primes_cpu, exact, bits, use_corr);
 }
 
 // out[b,m,n] = A[b,m,k] @ B[b,n,k]^T.   fp64_emu_cuda/fp64_emu.cu:1637-1662
@@ -130,13 +138,7 @@ void fp64_emu_bmm(at::Tensor& out, const at::Tensor& A, const at::Tensor& B,
   TORCH_CHECK(B.size(0) == batch && B.size(2) == K, "expect B as [batch, N, K]");
   check_out(out, A, {batch, M, N}, "out f64 [batch,M,N]");
   TORCH_CHECK(K <= kMaxKDeep, "K bound: 128 segments of 65536");
-  const c10::DeviceGuard guard(A.device());
-  const std::vector<int32_t> pv = primes_vec(primes_cpu);
-  const int P = (int)pv.size();
-  at::Tensor ws = workspace(A, fp64emu_workspace_size(batch, M, N, K, P, use_corr));
-  check_status(fp64emu_bmm(out.data_ptr<double>(), A.data_ptr<double>(), B.data_ptr<double>(),
-                           batch, M, N, K, pv.data(), nullptr, nullptr, P, exact, bits, use_corr,
-                           ws.data_ptr(), (size_t)ws.numel(), current_stream(A)));
+  product(out, A, B, batch, M, N, K, false, primes_cpu, exact, bits, use_corr);
 }
 
 // out[b,m,n] = A[b,m,k] @ Bt[b,k,n].   fp64_emu_cuda/fp64_emu.cu:1665-1686
@@ -151,14 +153,7 @@ void fp64_emu_bmm_nt(at::Tensor& out, const at::Tensor& A, const at::Tensor& Bt,
   TORCH_CHECK(Bt.size(0) == batch && Bt.size(1) == K, "expect Bt as [batch, K, N]");
   check_out(out, A, {batch, M, N}, "out f64 [batch,M,N]");
   TORCH_CHECK(K <= kMaxKSingle, "K bound for int32 modular GEMM");
-  const c10::DeviceGuard guard(A.device());
-  const std::vector<int32_t> pv = primes_vec(primes_cpu);
-  const int P = (int)pv.size();
-  at::Tensor ws = workspace(A, fp64emu_workspace_size(batch, M, N, K, P, use_corr));
-  check_status(fp64emu_bmm_nt(out.data_ptr<double>(), A.data_ptr<double>(),
-                              Bt.data_ptr<double>(), batch, M, N, K, pv.data(), nullptr, nullptr,
-                              P, exact, bits, use_corr, ws.data_ptr(), (size_t)ws.numel(),
-                              current_stream(A)));
+  product(out, A, Bt, batch, M, N, K, true, primes_cpu, exact, bits, use_corr);
 }
 
 // mm with phase times [scale+extract, gemms, marker, reconstruct] in ms.

@@ -24,7 +24,7 @@ EXPORTS = ("fp64emu_maxp", "fp64emu_last_error", "fp64emu_workspace_size",
            "fp64emu_workspace_size_min", "fp64emu_mm",
            "fp64emu_mm_nt", "fp64emu_bmm", "fp64emu_bmm_nt", "fp64emu_mm_timed",
            "fp64emu_mm_nt_events", "fp64emu_bmm_nt_events", "fp64emu_mm_nt_noalloc",
-           "fp64emu_layout",
+           "fp64emu_product_workspace", "fp64emu_product", "fp64emu_layout",
            "fp64emu_ddgemm_nt", "fp64emu_probe_mfma", "fp64emu_probe_stream")
 
 NOALLOC_SCRATCH_BYTES = 64 << 20   # FP64EMU_NOALLOC_SCRATCH_BYTES
@@ -50,6 +50,14 @@ class Layout(ctypes.Structure):
         return {name: getattr(self, name) for name, _ in self._fields_}
 
 
+class Product(ctypes.Structure):
+    """Mirror of fp64emu_product_t."""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("out", "A", "B")] + [
+        (n, ctypes.c_int64) for n in ("batch", "M", "N", "K")] + [
+            ("b_kn", ctypes.c_int), ("primes", ctypes.c_void_p), ("nprimes", ctypes.c_int),
+            ("exact", ctypes.c_int), ("bits", ctypes.c_int64), ("use_corr", ctypes.c_int)]
+
+
 _LIB = None
 
 
@@ -65,6 +73,10 @@ def lib():
     L.fp64emu_workspace_size.restype = sz
     L.fp64emu_workspace_size_min.argtypes = [i64, i64, i64, i64, i32, i32]
     L.fp64emu_workspace_size_min.restype = sz
+    L.fp64emu_product_workspace.argtypes = [ctypes.POINTER(Product)]
+    L.fp64emu_product_workspace.restype = sz
+    L.fp64emu_product.argtypes = [ctypes.POINTER(Product), vp, sz, vp]
+    L.fp64emu_product.restype = i32
     mm_args = [vp, vp, vp, i64, i64, i64, vp, vp, vp, i32, i32, i64, i32, vp, sz, vp]
     for name in ("fp64emu_mm", "fp64emu_mm_nt"):
         getattr(L, name).argtypes = mm_args
@@ -120,6 +132,32 @@ def workspace_size_min(batch, M, N, K, nprimes, use_corr):
 
 def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def product(kind, A, B, primes, exact=True, bits=53, use_corr=True, fill=None):
+    """fp64emu_product on checked device tensors: the call of the torch ops.
+    `fill`: a byte to fill the workspace with first."""
+    primes = np.ascontiguousarray(np.asarray(primes, dtype=np.int32))
+    batched, nt = kind in ("bmm", "bmm_nt"), kind.endswith("_nt")
+    if A.dim() != (3 if batched else 2) or B.dim() != A.dim() or (batched and B.shape[0] != A.shape[0]):
+        raise ValueError(f"{kind}: A {tuple(A.shape)} against B {tuple(B.shape)}")
+    batch = A.shape[0] if batched else 1
+    M, K = A.shape[-2:]
+    KB, N = (B.shape[-2], B.shape[-1]) if nt else (B.shape[-1], B.shape[-2])
+    if KB != K:
+        raise ValueError(f"{kind}: K of A is {K}, of B {KB}")
+    for name, t in (("A", A), ("B", B)):
+        if t.dtype != torch.float64 or not t.is_contiguous() or t.device != A.device:
+            raise ValueError(f"{kind}: {name} must be contiguous float64 on {A.device}")
+    out = torch.empty((batch, M, N) if batched else (M, N), dtype=torch.float64, device=A.device)
+    p = Product(out.data_ptr(), A.data_ptr(), B.data_ptr(), batch, M, N, K, int(nt),
+                primes.ctypes.data, primes.size, int(bool(exact)), int(bits), int(bool(use_corr)))
+    n = lib().fp64emu_product_workspace(ctypes.byref(p))
+    ws = torch.empty(max(int(n), 1), dtype=torch.uint8, device=A.device)
+    if fill is not None:
+        ws.fill_(fill)
+    _check(lib().fp64emu_product(ctypes.byref(p), ws.data_ptr(), ws.numel(), _stream()))
+    return out
 
 
 def run(kind, A, B, primes, exact=True, bits=53, use_corr=True, out=None, ws=None, fill=None):

@@ -157,6 +157,31 @@ int fp64emu_mm_nt_noalloc(double* out, const double* A, const double* Bt, int64_
                           const int64_t* mu, int nprimes, int exact, int64_t bits,
                           int use_corr, fp64emu_stream_t stream);
 
+/* One product in its quickest form, for callers that only want the result:
+ * the entry points above leave every stage of the call in the workspace (the
+ * map below), this one leaves nothing defined there and may lay it out and
+ * split the work differently.  Results are bit-identical.  b_kn: B given as
+ * [K, N] per member (the _nt calls), else [N, K].  No reference counterpart. */
+typedef struct {
+  double* out;             /* [batch, M, N] */
+  const double* A;         /* [batch, M, K] */
+  const double* B;
+  int64_t batch, M, N, K;
+  int b_kn;
+  const int32_t* primes;   /* host */
+  int nprimes, exact;
+  int64_t bits;
+  int use_corr;
+} fp64emu_product_t;
+
+/* Workspace of fp64emu_product (out, A and B may be NULL here).  On a shorter
+ * one the call runs as the entry points above would, down to
+ * fp64emu_workspace_size_min(). */
+size_t fp64emu_product_workspace(const fp64emu_product_t* p);
+
+int fp64emu_product(const fp64emu_product_t* p, void* workspace, size_t workspace_bytes,
+                    fp64emu_stream_t stream);
+
 /* ---- Workspace map (inspection of intermediates; no reference
  * counterpart: the reference's scratch is private torch tensors).  After a
  * call, the workspace holds that call's sizing outputs, operand planes,
