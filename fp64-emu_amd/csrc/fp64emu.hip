@@ -23,10 +23,12 @@
 //                  slots to balanced int8 and stores correction slots as
 //                  raw int32.
 //   4. reconstruct reconstruct_kernel: the exact combine of the usual plans
-//                  by remainder weights in three exact float64 slices (crt4),
+//                  by remainder weights in three exact float64 slices (crt_values),
 //                  otherwise balanced Garner digits with v_dot4_i32_i8 and
 //                  grouped Horner; the correction joins exactly, one
 //                  rounding, rescale.
+// Shallow products that need no stage kept (fp64emu_product) take stages 3 and
+// 4 in one launch, fused_kernel.
 //
 // The arithmetic each stage computes follows fp64_emu_cuda/fp64_emu.cu of the
 // reference (line citations at each kernel); the data layouts, launch shapes
@@ -556,6 +558,52 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
                        ? round_up(std::max<int64_t>(N, 1), 128) : L->Np;
 }
 
+// Fused products (fused_kernel): which tile the launch takes.  Against the
+// staged GEMM and reconstruction, a fused group loads its operands from L2 or
+// beyond with little reuse (a 64 x 64 tile reads 32 bytes an output and k-step
+// over 16 slots, a 256 x 256 tile 8), and saves the planes between (36 bytes an
+// output) and a launch.  So it pays for shallow products, and for deeper ones
+// only while they leave the chip idle.  Whole calls, staged / 32 x 32 / 64 x 32
+// / 64 x 64, us (mm or bmm, 14 + correction):
+//   64^3            21.1  17.6  18.8  22.8    1024^2 x 256    41.0  34.4  34.5  32.5
+//   128^2 x 512     24.7  22.2  25.7  31.0    1024^3          59.8  65.9  59.3  49.6
+//   128^2 x 1024    25.0  27.9  35.3  43.0    1024^2 x 2048   87.3   115  97.0  79.3
+//   256^2 x 1024    35.8  31.7  37.6  44.0    2000^2 x 512     101   110  97.7  95.9
+//   256^2 x 2048    38.3  43.1  52.6  64.2    2000^2 x 1000    132   200   174   143
+//   512^3           31.8  27.2  30.7  35.4    3000^2 x 256     145   129   120   145
+//   512^2 x 4096    78.4  73.7  97.8   119    64 x 256^3       136   114   108   118
+//   768^3           50.9  48.4  47.6  44.8    8 x 512^2 x 1024 121   138   123   108
+//   768^2 x 1536    64.6  74.3  72.6  64.1    16 x 512^3       138   141   128   123
+//   1500^2 x 256    58.0  50.1  51.0  58.8    32 x 512^3       267   315   290   301
+//   1500^2 x 700    83.4  97.8  88.0  90.3    64 x 512^2 x 128 263   240   201   249
+enum FusedTile { kFusedNone, kFused32x32, kFused64x32, kFused64x64 };
+
+FusedTile fused_tile(const fp64emu_layout_t& L) {
+  // Compiled for the planner's modulus counts at these depths; the fused
+  // correction's int32 bound; 32-bit offsets inside a member's planes.
+  if (L.deep || L.nchunk != 1 || (L.nprimes != 13 && L.nprimes != 14)) return kFusedNone;
+  if (L.memberA_bytes > 0xFFFFFFFFll || L.memberB_bytes > 0xFFFFFFFFll || L.K > kMaxKFusedCorr) return kFusedNone;
+  const int64_t nkt = L.Kp / kTileK;
+  auto tiles = [&](int64_t r, int64_t c) { return L.batch * ((L.M + r - 1) / r) * ((L.N + c - 1) / c); };
+  const int64_t t32 = tiles(32, 32), t64 = tiles(64, 64);
+  if (t32 <= kCUs)   // under a tile per CU; few and deep, the staged K-split spreads them wider
+    return nkt <= std::max<int64_t>(8, t32 / 4) ? kFused32x32 : kFusedNone;
+  if (t64 <= kCUs) {   // one round of the large tile, or (few of those) up to two of the small
+    if (nkt > 32) return kFusedNone;
+    return t64 > kCUs / 2 ? kFused64x64 : kFused32x32;
+  }
+  if (nkt <= 6) return kFused64x32;
+  const int64_t rounds = (t64 + kCUs - 1) / kCUs;
+  if (nkt <= 8 ? rounds <= 4 : nkt <= 16 && rounds <= 2 && t64 * 10 >= rounds * kCUs * 9) return kFused64x64;
+  return kFusedNone;
+}
+
+bool default_list(const int32_t* primes, int P) {
+  for (int t = 0; t < P; ++t)
+    if (primes[t] != kDefaultModuli[t]) return false;
+  return true;
+}
+
 // The layout of fp64emu_product, which leaves no stage for inspection: rows
 // past the operands' last 64-row group are never written (a GEMM output
 // depends on its own row and column alone, and the reconstruction reads the
@@ -564,7 +612,7 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
 constexpr size_t kWholeKBytes = (size_t)24 << 30;
 
 void make_product_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool corr,
-                         fp64emu_layout_t* L) {
+                         const int32_t* primes, FusedTile* fused, fp64emu_layout_t* L) {
   bool whole = whole_k_possible(K);
   make_layout(batch, M, N, K, P, corr, L, 1, whole);
   if (whole && L->total > kWholeKBytes) {
@@ -573,6 +621,8 @@ void make_product_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, 
   }
   L->ext_rowsA = round_up(std::max<int64_t>(M, 1), 64);
   L->ext_rowsB = round_up(std::max<int64_t>(N, 1), 64);
+  *fused = default_list(primes, P) ? fused_tile(*L) : kFusedNone;
+  if (*fused != kFusedNone) L->total = L->off_res8;   // no residue or correction planes
 }
 
 // ---------------------------------------------------------------------------
@@ -2491,7 +2541,7 @@ modgemm_split_x_kernel(GemmArgs g) {
 // Reconstruction.  Per output element, X from its residues, the correction
 // (corr1 + corr2) 2^(be - 15), one rounding to double, ldexp by -(sftA + sftB).
 // The exact combine of 12 to 15 default moduli sums remainder weights in
-// float64 (crt4); every other call takes balanced Garner digits
+// float64 (crt_values); every other call takes balanced Garner digits
 //   d_t = bal((r_t - sum_{u<t} d_u (M_u mod p_t)) (M_t mod p_t)^-1 mod p_t)
 // with the O(P^2) inner products as v_dot4_i32_i8 over packed digits; Horner
 // per group of 7 moduli (the first four steps of a group in int32: a balanced
@@ -2723,24 +2773,24 @@ __host__ __device__ __forceinline__ double crt_combine(double s1, double s2, dou
   return ldexp(h2 + yo, sh);
 }
 
-// Four elements' values from their residues r(t, e) (any representatives, or
+// kE elements' values from their residues r(t, e) (any representatives, or
 // sums of representatives: crt_exact), correction sums cv and shifts.
-template <int kP, typename R>
-__device__ __forceinline__ void crt4(const R& r, const double (&cv)[4], const int cshift,
-                                     const int (&sh)[4], double (&val)[4]) {
+template <int kP, int kE, typename R>
+__device__ __forceinline__ void crt_values(const R& r, const double (&cv)[kE], const int cshift,
+                                           const int (&sh)[kE], double (&val)[kE]) {
   constexpr CrtTab T = crt_tables(kP);
-  double s1[4] = {0.0, 0.0, 0.0, 0.0}, s2[4] = {0.0, 0.0, 0.0, 0.0}, s3[4] = {0.0, 0.0, 0.0, 0.0};
+  double s1[kE] = {}, s2[kE] = {}, s3[kE] = {};
 #pragma unroll
   for (int t = 0; t < kP; ++t)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < kE; ++e) {
       const double d = (double)r(t, e);
       s1[e] = fma(d, T.w[0][t], s1[e]);
       s2[e] = fma(d, T.w[1][t], s2[e]);
       s3[e] = fma(d, T.w[2][t], s3[e]);
     }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) val[e] = crt_combine<kP>(s1[e], s2[e], s3[e], cv[e], cshift, sh[e]);
+  for (int e = 0; e < kE; ++e) val[e] = crt_combine<kP>(s1[e], s2[e], s3[e], cv[e], cshift, sh[e]);
 }
 
 // One element's value from its Horner group values a0, a1, a2 (ng of them
@@ -3068,7 +3118,7 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
         double val[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) sh[e] = -(sai[e] + sj);
-        crt4<kP>([&](int t, int e) { return sums[t][e]; }, cv, cshift, sh, val);
+        crt_values<kP, 4>([&](int t, int e) { return sums[t][e]; }, cv, cshift, sh, val);
         store4(val);
         return;
       }
@@ -3106,7 +3156,7 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
     for (int e = 0; e < 4; ++e) sh[e] = -(sai[e] + sj);
     double val[4];
     if constexpr (kCrt) {
-      crt4<kP>([&](int t, int e) { return (int)(int8_t)(uint8_t)(w[t] >> (8 * e)); }, cv, cshift, sh, val);
+      crt_values<kP, 4>([&](int t, int e) { return (int)(int8_t)(uint8_t)(w[t] >> (8 * e)); }, cv, cshift, sh, val);
     } else {
       reconstruct4<kExact, kP>(w, cv, cshift, sh, val);
     }
@@ -3216,6 +3266,219 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
     store_at<double>(oblk + e * a.N, olane,
                      combine_groups<kExact>(ag[e][0], ag[e][1], ag[e][2], ng, false, tab_m64(0), tab_m64(1),
                                             (int64_t)cv[e], cshift, -(sai[e] + sj)));
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Modular GEMM and reconstruction in one kernel, for shallow products
+// (fused_tile): a group takes one output tile of 16 kTM x 16 kTN through every
+// slot and reconstructs it, so that no residue or correction plane is written
+// and read back (36 bytes an output at 14 moduli against the 8 of the result)
+// and the call is one launch shorter.
+//
+// The eight waves split the slots, not the tile: one takes the correction (two
+// residue slots' worth of k-steps) and the others two residue slots each, at
+// 14 moduli.  A wave shares no operand with the others, so it loads its
+// fragments from the planes straight into registers, kD k-steps ahead, with no
+// LDS ring and no barrier until the reconstruction: these products are bound by
+// the latency of plane reads that miss the L2 (~1.5 us), and every wave keeps
+// kD stages of its own in flight.  A slot's residues go to LDS as the
+// reconstruction's words (a lane's 4 values of a 16 x 16 accumulator block).
+
+typedef __amdgpu_buffer_rsrc_t BufferSrc;
+
+// A buffer resource over `bytes` bytes at p (raw; reads past its end return 0):
+// a load's address is its base, a per-lane offset that never changes and a
+// scalar offset, without vector address arithmetic.
+__device__ __forceinline__ BufferSrc buffer_src(const int8_t* p, uint32_t bytes) {
+  const uint64_t v = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<int8_t*>(((uint64_t)hi << 32) | lo), 0,
+                                           __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+
+template <int kOff>
+__device__ __forceinline__ v4i buffer_load16(BufferSrc src, uint32_t lane_off, uint32_t off) {
+  static_assert(kOff >= 0 && kOff < 4096, "buffer_load: offset outside its 12-bit field");
+  typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+  const v4u v = __builtin_amdgcn_raw_buffer_load_b128(src, (int)lane_off + kOff,
+                                                      __builtin_amdgcn_readfirstlane((int)off), 0);
+  return __builtin_bit_cast(v4i, v);
+}
+
+struct FusedArgs {
+  const int8_t* A;
+  const int8_t* B;
+  double* out;
+  const int16_t* sftA;
+  const int16_t* sftB;
+  const int* bits_eff;
+  int64_t memberA, memberB, planeA, planeB;
+  int64_t M, N;
+  uint32_t total;      // groups: batch x TM x TN
+  int nkt;             // k tiles of a residue plane
+  int TM, TN;          // output tiles per member
+  int use_corr;
+  FastDiv div_tiles;   // by TM TN
+  FastDiv div_grp;     // by 8 TN (8 row tiles, every column tile)
+};
+
+constexpr int kFusedThreads = 512;
+constexpr int kFusedWaves = kFusedThreads / 64;
+
+// kD: k-steps in flight per wave; kWavesPerSimd: the register budget.
+template <bool kExact, int kP, int kTM, int kTN, int kD, int kWavesPerSimd>
+__global__ void __launch_bounds__(kFusedThreads, kWavesPerSimd)
+fused_kernel(FusedArgs g) {
+  constexpr int kBlk = kTM * kTN;
+  __shared__ uint32_t s_res[kP][kBlk][64];
+  __shared__ v4i s_corr[kBlk][64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // XCD-aware order: group i runs on XCD i % 8; of each full chunk of 256
+  // groups XCD x takes tiles 32 x .. 32 x + 31, which share operand panels in
+  // its L2.
+  const uint32_t i = blockIdx.x;
+  const uint32_t L = (i >> 8) < (g.total >> 8) ? (i & ~255u) + (i & 7) * 32 + ((i & 255) >> 3) : i;
+  const uint32_t b = g.div_tiles.div(L);
+  const uint32_t tile = L - b * g.div_tiles.d;
+  // Grouped tile order: 8 row tiles per group, column-major inside.
+  const uint32_t grp = g.div_grp.div(tile);
+  const uint32_t within = tile - grp * g.div_grp.d;
+  const uint32_t gm = min((uint32_t)g.TM - 8 * grp, 8u);
+  const uint32_t nt = gm == 8 ? within >> 3 : within / gm;
+  const uint32_t mt = 8 * grp + within - nt * gm;
+
+  // The thread's outputs in the reconstruction: kE values of a word of blocks
+  // blk0, blk0 + 8, .. (from value 2 sub).
+  constexpr int kE = kExact && kBlk == 4 ? 2 : 4;   // values a thread and iteration
+  const int sub = kE == 2 ? wave & 1 : 0;
+  const int blk0 = kE == 2 ? wave >> 1 : wave;
+  const int nkt = g.nkt;
+
+  const BufferSrc srcA = buffer_src(g.A + b * g.memberA, (uint32_t)g.memberA);
+  const BufferSrc srcB = buffer_src(g.B + b * g.memberB, (uint32_t)g.memberB);
+  const uint32_t loff = (uint32_t)lane * 16;
+  const uint32_t fa = mt * kTM, fb = nt * kTN;
+  const uint32_t rowA = (fa >> 4) * (uint32_t)nkt, rowB = (fb >> 4) * (uint32_t)nkt;   // plane tiles
+  const uint32_t inA = (fa & 15) * kFragBytes, inB = (fb & 15) * kFragBytes;
+
+  // Slots of a wave: with a correction (2 nkt k-steps) the last wave takes it
+  // and wave w moduli w, w + 7; without one, moduli w, w + 8.
+  const bool corr = g.use_corr != 0;
+  const bool corr_wave = corr && wave == kFusedWaves - 1;
+  const int t0 = corr_wave ? kP : wave;
+  const int tstep = corr ? kFusedWaves - 1 : kFusedWaves;
+  const int n = corr_wave ? 2 * nkt : nkt;   // k-steps of each of the wave's slots
+
+  v4i FA[kD][kTM], FB[kD][kTN];
+  v4i acc[kTM][kTN];
+  auto load = [&](v4i (&A)[kTM], v4i (&B)[kTN], const int t, const int k) {
+    const uint32_t r = corr_wave ? 2 : 1;
+    const uint32_t oa = (uint32_t)t * (uint32_t)g.planeA + (r * rowA + (uint32_t)k) * kTileBytes + inA;
+    const uint32_t ob = (uint32_t)t * (uint32_t)g.planeB + (r * rowB + (uint32_t)k) * kTileBytes + inB;
+    if constexpr (kTM > 0) A[0] = buffer_load16<0>(srcA, loff, oa);
+    if constexpr (kTM > 1) A[1] = buffer_load16<1024>(srcA, loff, oa);
+    if constexpr (kTM > 2) A[2] = buffer_load16<2048>(srcA, loff, oa);
+    if constexpr (kTM > 3) A[3] = buffer_load16<3072>(srcA, loff, oa);
+    if constexpr (kTN > 0) B[0] = buffer_load16<0>(srcB, loff, ob);
+    if constexpr (kTN > 1) B[1] = buffer_load16<1024>(srcB, loff, ob);
+    if constexpr (kTN > 2) B[2] = buffer_load16<2048>(srcB, loff, ob);
+    if constexpr (kTN > 3) B[3] = buffer_load16<3072>(srcB, loff, ob);
+  };
+  auto mma = [&](const v4i (&A)[kTM], const v4i (&B)[kTN]) {
+#pragma unroll
+    for (int x = 0; x < kTM; ++x)
+#pragma unroll
+      for (int yy = 0; yy < kTN; ++yy) {
+        const int y = (x & 1) ? kTN - 1 - yy : yy;
+        acc[x][y] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[x], B[y], acc[x][y], 0, 0, 0);
+      }
+  };
+#pragma unroll
+  for (int d = 0; d < kD; ++d) load(FA[d], FB[d], min(t0, kP), min(d, n - 1));
+
+  const int be = g.bits_eff[0], grow = g.bits_eff[1];
+  const int64_t om0 = (int64_t)mt * (16 * kTM) + 4 * (lane >> 4) + 2 * sub, on0 = (int64_t)nt * (16 * kTN) + (lane & 15);
+
+  for (int t = t0; t < kP || (corr_wave && t == kP); t += tstep) {
+#pragma unroll
+    for (int x = 0; x < kTM; ++x)
+#pragma unroll
+      for (int y = 0; y < kTN; ++y) acc[x][y] = v4i{0, 0, 0, 0};
+    const int tc = min(t, kP - 1);
+    const double ip = kDefaultTab.invp[tc];
+    const int negp = -kDefaultTab.p[tc];
+    int k = 0;
+    for (; k + kD < n; k += kD) {
+#pragma unroll
+      for (int d = 0; d < kD; ++d) {
+        mma(FA[d], FB[d]);
+        load(FA[d], FB[d], t, min(k + d + kD, n - 1));
+      }
+    }
+    // The last 1 .. kD k-steps; then the next slot's first ones.
+#pragma unroll
+    for (int d = 0; d < kD; ++d)
+      if (k + d < n) mma(FA[d], FB[d]);
+    if (t + tstep < kP && !corr_wave) {
+#pragma unroll
+      for (int d = 0; d < kD; ++d) load(FA[d], FB[d], t + tstep, min(d, n - 1));
+    }
+    if (corr_wave) {
+#pragma unroll
+      for (int x = 0; x < kTM; ++x)
+#pragma unroll
+        for (int y = 0; y < kTN; ++y) s_corr[x * kTN + y][lane] = acc[x][y];
+    } else {
+#pragma unroll
+      for (int x = 0; x < kTM; ++x)
+#pragma unroll
+        for (int y = 0; y < kTN; ++y) {
+          const v4i a = acc[x][y];
+          int q[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q[e] = __double2loint(fma((double)a[e], ip, kMagic));
+          s_res[t][x * kTN + y][lane] = pack_bytes(__mul24(q[0], negp) + a[0], __mul24(q[1], negp) + a[1],
+                                                   __mul24(q[2], negp) + a[2], __mul24(q[3], negp) + a[3]);
+        }
+    }
+  }
+  __syncthreads();
+
+  // Reconstruction of blocks blk0, blk0 + 8, ..
+  const int16_t* const sA = g.sftA + b * g.M;
+  const int16_t* const sB = g.sftB + b * g.N;
+  double* const out = g.out + (int64_t)b * g.M * g.N;
+#pragma unroll 1
+  for (int blk = blk0; blk < kBlk; blk += kFusedWaves) {
+    const int64_t m = om0 + 16 * (blk / kTN), nn = on0 + 16 * (blk % kTN);
+    if (m >= g.M || nn >= g.N) continue;
+    uint32_t w[kMaxP];
+#pragma unroll
+    for (int t = 0; t < kP; ++t) w[t] = s_res[t][blk][lane];
+    v4i c = v4i{0, 0, 0, 0};
+    if (corr) c = s_corr[blk][lane];
+    const int sj = (int)sB[nn] + 2 * grow;
+    int sh[kE];
+    std::conditional_t<kExact, double, int64_t> cv[kE];
+#pragma unroll
+    for (int e = 0; e < kE; ++e) {
+      sh[e] = -((int)sA[min(m + e, g.M - 1)] + sj);
+      cv[e] = kE == 2 ? (sub ? c[2 + e] : c[e]) : c[e];
+    }
+    double val[kE];
+    if constexpr (kExact)
+      crt_values<kP, kE>([&](int t, int e) { return (int)(int8_t)(uint8_t)(w[t] >> (16 * sub + 8 * e)); }, cv,
+                         be - 15, sh, val);
+    else
+      reconstruct4<kExact, kP>(w, cv, be - 15, sh, val);
+    double* const o = out + m * g.N + nn;
+#pragma unroll
+    for (int e = 0; e < kE; ++e)
+      if (m + e < g.M) o[e * g.N] = val[e];
   }
 }
 
@@ -3548,6 +3811,26 @@ void launch_reconstruct(bool exact, int P, unsigned grid, hipStream_t s, const R
   }
 }
 
+template <bool kExact, int kP>
+void launch_fused_t(FusedTile tile, unsigned grid, hipStream_t s, const FusedArgs& g) {
+  if (tile == kFused64x64)
+    hipLaunchKernelGGL((fused_kernel<kExact, kP, 4, 4, 4, 2>), dim3(grid), dim3(kFusedThreads), 0, s, g);
+  else if (tile == kFused64x32)
+    hipLaunchKernelGGL((fused_kernel<kExact, kP, 4, 2, 3, 4>), dim3(grid), dim3(kFusedThreads), 0, s, g);
+  else
+    hipLaunchKernelGGL((fused_kernel<kExact, kP, 2, 2, 4, 4>), dim3(grid), dim3(kFusedThreads), 0, s, g);
+}
+
+void launch_fused(FusedTile tile, bool exact, int P, unsigned grid, hipStream_t s, const FusedArgs& g) {
+  if (P == 14) {
+    if (exact) launch_fused_t<true, 14>(tile, grid, s, g);
+    else launch_fused_t<false, 14>(tile, grid, s, g);
+  } else {
+    if (exact) launch_fused_t<true, 13>(tile, grid, s, g);
+    else launch_fused_t<false, 13>(tile, grid, s, g);
+  }
+}
+
 int run(const Call& c) {
   if (int st = validate_primes(c.primes, c.P)) return st;
   if (c.bits < 16 || c.bits > 53) return fail(FP64EMU_EINVAL, "bits must be in [16, 53]");
@@ -3557,9 +3840,13 @@ int run(const Call& c) {
     return fail(FP64EMU_EINVAL, "K bound for int32 modular GEMM");
   if (c.K > kMaxKDeep) return fail(FP64EMU_EINVAL, "K bound: 128 segments of 65536");
   fp64emu_layout_t L;
-  if (c.product) make_product_layout(c.batch, c.M, c.N, c.K, c.P, c.corr, &L);
+  FusedTile fused = kFusedNone;
+  if (c.product) make_product_layout(c.batch, c.M, c.N, c.K, c.P, c.corr, c.primes, &fused, &L);
   // (A product on a shorter workspace runs as the other entry points do.)
-  if (!c.product || c.ws_bytes < L.total) make_layout(c.batch, c.M, c.N, c.K, c.P, c.corr, &L);
+  if (!c.product || c.ws_bytes < L.total) {
+    fused = kFusedNone;
+    make_layout(c.batch, c.M, c.N, c.K, c.P, c.corr, &L);
+  }
   const hipStream_t s = c.stream;
   if (c.ev) {
     if (int st = check_hip(hipEventRecord(c.ev[0], s), "hipEventRecord")) return st;
@@ -3681,7 +3968,9 @@ int run(const Call& c) {
             : (group ? MF : (MF + kRowsPerBlock - 1) / kRowsPerBlock) + (NF + kThreads - 1) / kThreads * nslab;
     const int64_t extraction = c.batch * (L.ext_rowsA / 64 + L.ext_rowsB / 64) * (L.Kp / kTileK);
     const int64_t recon = c.batch * ((std::min<int64_t>(L.chunk_rows, c.M) + 15) / 16) * ((c.N + 63) / 64);
-    for (int64_t gsz : {sizing, extraction, ga.total, recon})
+    // (Fused groups, twice kThreads wide, of at least 32 x 32 outputs.)
+    const int64_t tiles = fused == kFusedNone ? 0 : 2 * c.batch * ((c.M + 31) / 32) * ((c.N + 31) / 32);
+    for (int64_t gsz : {sizing, extraction, ga.total, recon, tiles})
       if (gsz > limit) return fail(FP64EMU_EINVAL, "problem too large for one launch");
   }
 
@@ -3774,6 +4063,23 @@ int run(const Call& c) {
       }
       if (c.ev) {
         if (int st = check_hip(hipEventRecord(c.ev[1], s), "hipEventRecord")) return st;
+      }
+      if (fused != kFusedNone) {
+        const int64_t rows = fused == kFused32x32 ? 32 : 64, cols = fused == kFused64x64 ? 64 : 32;
+        FusedArgs fa;
+        fa.A = planesA; fa.B = planesB; fa.out = c.out;
+        fa.sftA = sftA; fa.sftB = sftB; fa.bits_eff = bits_eff;
+        fa.memberA = L.memberA_bytes; fa.memberB = L.memberB_bytes;
+        fa.planeA = L.planeA_bytes; fa.planeB = L.planeB_bytes;
+        fa.M = c.M; fa.N = c.N;
+        fa.nkt = (int)nkt;
+        fa.TM = (int)((c.M + rows - 1) / rows); fa.TN = (int)((c.N + cols - 1) / cols);
+        fa.total = (uint32_t)(c.batch * fa.TM * fa.TN);
+        fa.use_corr = c.corr ? 1 : 0;
+        fa.div_tiles = make_fastdiv((int64_t)fa.TM * fa.TN);
+        fa.div_grp = make_fastdiv((int64_t)8 * fa.TN);
+        launch_fused(fused, c.exact, c.P, fa.total, s, fa);
+        return check_hip(hipGetLastError(), "kernel launch");
       }
       ga.nkt = (int)nkt;
       ga.first = seg == 0 ? 1 : 0;
@@ -3927,10 +4233,12 @@ size_t fp64emu_workspace_size_min(int64_t batch, int64_t M, int64_t N, int64_t K
 }
 
 size_t fp64emu_product_workspace(const fp64emu_product_t* p) {
-  if (!p || p->batch < 0 || p->M < 0 || p->N < 0 || p->K < 0 || p->nprimes < 1 || p->nprimes > kMaxP)
+  if (!p || p->batch < 0 || p->M < 0 || p->N < 0 || p->K < 0 || p->nprimes < 1 || p->nprimes > kMaxP ||
+      !p->primes)
     return 0;
   fp64emu_layout_t L;
-  make_product_layout(p->batch, p->M, p->N, p->K, p->nprimes, p->use_corr != 0, &L);
+  FusedTile fused;
+  make_product_layout(p->batch, p->M, p->N, p->K, p->nprimes, p->use_corr != 0, p->primes, &fused, &L);
   return L.total;
 }
 

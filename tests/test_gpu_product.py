@@ -56,3 +56,34 @@ def test_whole_k(dev, kind, batch, M, N, K, P, corr, exact):
 ])
 def test_unpadded_rows(dev, kind, batch, M, N, K, P, corr):
     _check(dev, kind, batch, M, N, K, P, corr)
+
+
+# Fused GEMM and reconstruction: each tile (32 x 32, 64 x 32, 64 x 64), edges inside and
+# at fragments and tiles, one k-step, depths that are not a multiple of the steps in
+# flight, members, both combines, 13 and 14 moduli, with and without the correction.
+@pytest.mark.parametrize("kind,batch,M,N,K", [
+    ("mm", 1, 1, 1, 1), ("mm_nt", 1, 16, 17, 64), ("mm", 1, 33, 31, 65), ("bmm_nt", 3, 47, 50, 200),
+    ("mm_nt", 1, 512, 512, 64 * 17),                                           # 32 x 32, 256 tiles
+    ("bmm", 5, 400, 410, 3 * 64 + 5), ("bmm_nt", 40, 129, 200, 257),           # 64 x 32
+    ("mm", 1, 800, 900, 700), ("bmm_nt", 12, 500, 300, 500), ("mm_nt", 1, 1025, 1000, 1100),   # 64 x 64
+])
+@pytest.mark.parametrize("P,corr,exact", [(14, True, True), (13, False, True), (14, True, False), (13, True, False),
+                                          (14, False, True)])
+def test_fused(dev, kind, batch, M, N, K, P, corr, exact):
+    _check(dev, kind, batch, M, N, K, P, corr, exact)
+
+
+def test_fused_zero_and_nonfinite(dev):
+    """Zeros give +0; rows and columns holding infinities or NaN change only
+    what they change in the staged form (their values extract to 0 and the
+    width stays at 53 bits)."""
+    for special in (0.0, float("inf"), float("-inf"), float("nan"), 1e308, 5e-324):
+        print(f"case fused special {special}", flush=True)
+        A, B = _pair("mm", 1, 70, 90, 130, 9, dev)
+        A[3, 5] = special
+        A[7] = 0.0
+        B[:, 11] = special
+        got = capi.product("mm", A, B, O.PRIMES[:14])
+        ref, _, _ = capi.run("mm", A, B, O.PRIMES[:14])
+        torch.cuda.synchronize()
+        assert bits_equal(got.cpu().numpy(), ref.cpu().numpy())
