@@ -1122,8 +1122,8 @@ struct ExtractCore {
   int use_corr;
   int64_t nkt;       // Kp / 64
   int64_t planeA, planeB, memberA, memberB;
-  int64_t rgA, rgB;  // 64-row groups per member the GEMM reads (0: B not extracted)
-  int64_t rgA_data, rgB_data;   // those holding operand rows: ceil(M / 64), ceil(N / 64)
+  int64_t rgA, rgB;  // 4 kEl-row groups per member the GEMM reads (0: B not extracted)
+  int64_t rgA_data, rgB_data;   // those holding operand rows
   // Dividers of the work-group decomposition: by nkt, and by the row-group
   // count of each segment (A data, B data, A padding, B padding).
   FastDiv div_nkt, div_rg[4];
@@ -1150,17 +1150,32 @@ struct ExtractCore {
 template <bool kTab> struct ExtractArgs : ExtractCore { ModTables tab; };
 template <> struct ExtractArgs<false> : ExtractCore {};
 
+// kEl: elements (consecutive k) per lane.  16 in launches that fill the chip;
+// 4 in those of at most kSmallExtractGroups groups of 64 rows, whose waves
+// otherwise run their 16 elements' loads and 14 planes' arithmetic alone on a
+// SIMD (four times the waves, a quarter of the chain; dword stores).  16 / 4
+// elements, whole calls: 64^3 16.4 / 13.8 us, 256^3 19.5 / 16.5, 333 x 501 x
+// 777 34.7 / 33.0, 512^3 27.0 / 24.8, 768^3 (288 groups) 44.7 / 42.1; even at
+// 512 groups (1024^3 49.6 / 50.3, 512^2 x 2048 45.1 / 45.4), slower beyond
+// (64 x 256^3 108.5 / 114).
+constexpr int64_t kSmallExtractGroups = 384;
+
 // kDefault: the modulus list is a prefix of the default one, whose constants
 // the plane loop takes at compile time (no scalar load and wait per plane,
 // which dominated small launches); otherwise the tables of the arguments.
-template <bool kDefault>
+template <bool kDefault, int kEl>
 __global__ void __launch_bounds__(kThreads)
 extract_kernel(ExtractArgs<!kDefault> a) {
+  constexpr int kW = kEl / 4;   // packed residue words per lane and plane
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // The width pick, when this launch takes it: every wave reaches the
-  // block's barrier before any returns.
+  // block's barrier before any returns.  Small launches (kEl = 4) read the
+  // operand first, so that one round trip covers both (512^3 27.2 -> 27.0 us);
+  // in launches of many groups holding the operand across the barrier cost
+  // more (2000^3 211 -> 214 us).
   int pick_be = 0;
-  if (a.pick) {
+  auto width_pick = [&]() {
+    if (!a.pick) return;
     float ma, mb;
     block_max_lg_pair<kThreads>(a.lgA, a.nlgA, a.lgB, a.nlgB, ma, mb);
     pick_be = pick_width(ma, mb, a.log2M, a.bits);
@@ -1168,7 +1183,8 @@ extract_kernel(ExtractArgs<!kDefault> a) {
       a.bits_out[0] = pick_be;
       a.bits_out[1] = pick_be - a.bits;
     }
-  }
+  };
+  if constexpr (kEl == 16) width_pick();
   // Work groups: the row groups holding operand rows of A, then of B, then
   // the all-padding row groups of A and of B (zero stores only), so that the
   // work spreads evenly over the XCDs (group i runs on XCD i % 8) whatever
@@ -1211,11 +1227,13 @@ extract_kernel(ExtractArgs<!kDefault> a) {
   rg += rg_off;
   const int64_t R = isA ? a.M : a.N;
   const int64_t K = a.K;
-  // Wave w covers rows 64 rg + 16 w .. +16 and the whole k tile: one
+  // kEl = 16: wave w covers rows 64 rg + 16 w .. +16 and the whole k tile, one
   // 16 x 64 fragment, lane l = 16 (k / 16) + row % 16 holding 16 k.
-  const int64_t rblk = rg * 4 + wave;                            // 16-row block
+  // kEl = 4: the group covers 16 rows, wave w the 16 k of fragment lanes
+  // 16 w .. + 15, lane l row l % 16 and the k / 4 % 4 = l / 16 quarter of them.
+  const int64_t rblk = kEl == 16 ? rg * 4 + wave : rg;           // 16-row block
   const int64_t r = rblk * 16 + (lane & 15);                     // plane row (A row or B column)
-  const int64_t k0 = kt * kTileK + (lane >> 4) * 16;             // first of 16 k
+  const int64_t k0 = kt * kTileK + (kEl == 16 ? 0 : wave * 16) + (lane >> 4) * kEl;   // first of kEl k
   const bool rowok = r < R;
 
   // A fragment that is all padding (its 16 rows or its 64 k past the
@@ -1225,36 +1243,44 @@ extract_kernel(ExtractArgs<!kDefault> a) {
   const int64_t rt = rblk >> 4, fr = rblk & 15;
   const int64_t plane = isA ? a.planeA : a.planeB;
   int8_t* base = (isA ? a.planesA : a.planesB) + b * (isA ? a.memberA : a.memberB);
-  const int64_t off = (rt * nkt + kt) * kTileBytes + fr * kFragBytes + lane * 16;
-  if (__builtin_amdgcn_readfirstlane((int)(rblk * 16 >= R || kt * kTileK >= K))) {
-    const v4i z = v4i{0, 0, 0, 0};
-    for (int pi = 0; pi < P; ++pi) *reinterpret_cast<v4i*>(base + pi * plane + off) = z;
-    if (a.use_corr) {
-      int8_t* cb = base + (int64_t)P * plane;
-      const int64_t o1 = (rt * 2 * nkt + kt) * kTileBytes + fr * kFragBytes + lane * 16;
-      *reinterpret_cast<v4i*>(cb + o1) = z;
-      *reinterpret_cast<v4i*>(cb + o1 + nkt * kTileBytes) = z;
-    }
-    return;
-  }
+  const int in_frag = kEl == 16 ? lane * 16 : wave * 256 + (lane & 15) * 16 + (lane >> 4) * 4;
+  const int64_t off = (rt * nkt + kt) * kTileBytes + fr * kFragBytes + in_frag;
+  typedef std::conditional_t<kEl == 16, v4i, int> Words;
+  auto store_words = [&](int8_t* at, const uint32_t (&w)[kW]) {
+    if constexpr (kEl == 16) *reinterpret_cast<v4i*>(at) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+    else *reinterpret_cast<uint32_t*>(at) = w[0];
+  };
+  const bool padding = __builtin_amdgcn_readfirstlane((int)(rblk * 16 >= R || kt * kTileK >= K));
 
-  double x[16];
-  if (!rowok || k0 >= K) {
+  double x[kEl];
+  if (padding || !rowok || k0 >= K) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) x[j] = 0.0;
+    for (int j = 0; j < kEl; ++j) x[j] = 0.0;
   } else if (kn) {
     const double* __restrict__ src = a.B + (b * a.lda + a.k0 + k0) * a.N + r;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) x[j] = (k0 + j < K) ? src[(int64_t)j * a.N] : 0.0;
+    for (int j = 0; j < kEl; ++j) x[j] = (k0 + j < K) ? src[(int64_t)j * a.N] : 0.0;
   } else {
     const double* __restrict__ src = (isA ? a.A : a.B) + (b * R + r) * a.lda + a.k0 + k0;
-    if (k0 + 16 <= K) {
+    if (k0 + kEl <= K) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) x[j] = src[j];
+      for (int j = 0; j < kEl; ++j) x[j] = src[j];
     } else {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) x[j] = (k0 + j < K) ? src[j] : 0.0;
+      for (int j = 0; j < kEl; ++j) x[j] = (k0 + j < K) ? src[j] : 0.0;
     }
+  }
+  if constexpr (kEl != 16) width_pick();
+  if (padding) {
+    const Words z = {};
+    for (int pi = 0; pi < P; ++pi) *reinterpret_cast<Words*>(base + pi * plane + off) = z;
+    if (a.use_corr) {
+      int8_t* cb = base + (int64_t)P * plane;
+      const int64_t o1 = (rt * 2 * nkt + kt) * kTileBytes + fr * kFragBytes + in_frag;
+      *reinterpret_cast<Words*>(cb + o1) = z;
+      *reinterpret_cast<Words*>(cb + o1 + nkt * kTileBytes) = z;
+    }
+    return;
   }
 
   // Shift: per row of A / of B [N,K]; per column of B [K,N] -- one per lane.
@@ -1271,10 +1297,10 @@ extract_kernel(ExtractArgs<!kDefault> a) {
   // so the tie parity is unchanged.  td = +-Tu (|td| <= 2^53) splits as
   // th 2^31 + tl with th = RNE(td / 2^31), |th| <= 2^22, and |tl| <= 2^30,
   // both exact int32s.
-  int th[16], tl[16];
-  uint32_t hw[4] = {0u, 0u, 0u, 0u}, qw[4] = {0u, 0u, 0u, 0u};
+  int th[kEl], tl[kEl];
+  uint32_t hw[kW] = {}, qw[kW] = {};
 #pragma unroll
-  for (int jj = 0; jj < 16; ++jj) {
+  for (int jj = 0; jj < kEl; ++jj) {
     // Infinities and NaNs scale to 0, as the reference's integer split of
     // their encoding does (the shift that carries exponent 0x7FF is far past
     // 64 bits); every finite y is below 2^53.
@@ -1296,8 +1322,8 @@ extract_kernel(ExtractArgs<!kDefault> a) {
     tl[jj] = (int)fma(-hi, 2147483648.0, td);      // in [-2^30, 2^30]
   }
 
-  // One plane at a time: 16 residues -> one 16-byte chunk per lane, 1 KiB
-  // contiguous per wave.  v = th (2^31 mod p) + tl is an exact int32
+  // One plane at a time: kEl residues -> one kEl-byte chunk per lane, 64 kEl
+  // bytes contiguous per wave.  v = th (2^31 mod p) + tl is an exact int32
   // (|v| <= 2^21 p + 2^30 < 2^31) congruent to td; its balanced residue
   // v - p RNE(v / p) lies in [-p/2, p/2] (for odd p the quotient v RN(1/p) is
   // at most 2^-30 off v / p, which never comes within 1/(2p) of a
@@ -1315,9 +1341,9 @@ extract_kernel(ExtractArgs<!kDefault> a) {
     } else {
       pt = a.tab.p[pi]; c31 = a.tab.c31[pi]; ip = a.tab.invp[pi];
     }
-    uint32_t w4[4];
+    uint32_t w4[kW];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
+    for (int g = 0; g < kW; ++g) {
       int r[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
@@ -1333,8 +1359,7 @@ extract_kernel(ExtractArgs<!kDefault> a) {
       }
       w4[g] = pack_bytes(r[0], r[1], r[2], r[3]);
     }
-    *reinterpret_cast<v4i*>(base + pi * plane + off) =
-        v4i{(int)w4[0], (int)w4[1], (int)w4[2], (int)w4[3]};
+    store_words(base + pi * plane + off, w4);
   };
   if constexpr (kDefault) {
     // Every default modulus is 256 or odd, and >= 171.
@@ -1357,12 +1382,10 @@ extract_kernel(ExtractArgs<!kDefault> a) {
   if (a.use_corr) {
     // Correction plane: row tile stride 2*nkt tiles; A = [hi | q], B = [q | hi].
     int8_t* cb = base + (int64_t)P * plane;
-    const int64_t o1 = (rt * 2 * nkt + kt) * kTileBytes + fr * kFragBytes + lane * 16;
+    const int64_t o1 = (rt * 2 * nkt + kt) * kTileBytes + fr * kFragBytes + in_frag;
     const int64_t o2 = o1 + nkt * kTileBytes;
-    const v4i hv = v4i{(int)hw[0], (int)hw[1], (int)hw[2], (int)hw[3]};
-    const v4i qv = v4i{(int)qw[0], (int)qw[1], (int)qw[2], (int)qw[3]};
-    *reinterpret_cast<v4i*>(cb + o1) = isA ? hv : qv;
-    *reinterpret_cast<v4i*>(cb + o2) = isA ? qv : hv;
+    store_words(cb + o1, isA ? hw : qw);
+    store_words(cb + o2, isA ? qw : hw);
   }
 }
 
@@ -4010,7 +4033,9 @@ int run(const Call& c) {
     }
   }
   const float log2M = std::min(tab.log2M, 126.0f);
-  const int64_t ext_groups = c.batch * (L.ext_rowsA / 64 + L.ext_rowsB / 64) * (L.Kp / kTileK);
+  const int64_t groups64 = c.batch * (L.ext_rowsA / 64 + L.ext_rowsB / 64) * (L.Kp / kTileK);
+  const int64_t ext_rows = default_moduli && groups64 <= kSmallExtractGroups ? 16 : 64;   // rows of an extraction group
+  const int64_t ext_groups = groups64 * (64 / ext_rows);
   const bool pick_in_extract = L.nchunk == 1 && L.nseg == 1 && MF + NF <= kPickInExtractMax &&
                                (MF + NF) * (int64_t)sizeof(float) * ext_groups <= kPickInExtractBytes;
   if (!pick_in_extract)
@@ -4038,8 +4063,8 @@ int run(const Call& c) {
       ea.nkt = nkt;
       ea.planeA = L.planeA_bytes; ea.planeB = L.planeB_bytes;
       ea.memberA = L.memberA_bytes; ea.memberB = L.memberB_bytes;
-      ea.rgA = L.ext_rowsA / 64; ea.rgB = with_B ? L.ext_rowsB / 64 : 0;
-      ea.rgA_data = (Mc + 63) / 64; ea.rgB_data = with_B ? (c.N + 63) / 64 : 0;
+      ea.rgA = L.ext_rowsA / ext_rows; ea.rgB = with_B ? L.ext_rowsB / ext_rows : 0;
+      ea.rgA_data = (Mc + ext_rows - 1) / ext_rows; ea.rgB_data = with_B ? (c.N + ext_rows - 1) / ext_rows : 0;
       ea.div_nkt = make_fastdiv(nkt);
       ea.div_rg[0] = make_fastdiv(ea.rgA_data);
       ea.div_rg[1] = make_fastdiv(ea.rgB_data);
@@ -4054,12 +4079,15 @@ int run(const Call& c) {
       if (default_moduli) {
         ExtractArgs<false> ed;
         static_cast<ExtractCore&>(ed) = ea;
-        hipLaunchKernelGGL(extract_kernel<true>, dim3((unsigned)wg), dim3(kThreads), 0, s, ed);
+        if (ext_rows == 16)
+          hipLaunchKernelGGL((extract_kernel<true, 4>), dim3((unsigned)wg), dim3(kThreads), 0, s, ed);
+        else
+          hipLaunchKernelGGL((extract_kernel<true, 16>), dim3((unsigned)wg), dim3(kThreads), 0, s, ed);
       } else {
         ExtractArgs<true> eg;
         static_cast<ExtractCore&>(eg) = ea;
         eg.tab = tab;
-        hipLaunchKernelGGL(extract_kernel<false>, dim3((unsigned)wg), dim3(kThreads), 0, s, eg);
+        hipLaunchKernelGGL((extract_kernel<false, 16>), dim3((unsigned)wg), dim3(kThreads), 0, s, eg);
       }
       if (c.ev) {
         if (int st = check_hip(hipEventRecord(c.ev[1], s), "hipEventRecord")) return st;
