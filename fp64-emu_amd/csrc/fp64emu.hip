@@ -210,6 +210,31 @@ ModTables make_tables(const int32_t* primes, int P) {
   return T;
 }
 
+bool default_list(const int32_t* primes, int P) {
+  for (int t = 0; t < P; ++t)
+    if (primes[t] != kDefaultModuli[t]) return false;
+  return true;
+}
+
+// The tables of a modulus list (`own`: where a list outside the default one's
+// prefixes is computed).  The prefixes' tables are constants of the library,
+// computed on first use: the inverses and logarithms of 14 moduli took 3-4 us
+// of every call.
+const ModTables& call_tables(const int32_t* primes, int P, ModTables* own) {
+  if (!default_list(primes, P)) {
+    *own = make_tables(primes, P);
+    return *own;
+  }
+  struct Prefixes {
+    ModTables t[kMaxP + 1];
+    Prefixes() {
+      for (int n = 0; n <= kMaxP; ++n) t[n] = make_tables(kDefaultModuli, n);
+    }
+  };
+  static const Prefixes prefixes;
+  return prefixes.t[P];
+}
+
 // ---------------------------------------------------------------------------
 // Workspace map.
 constexpr size_t kAlign = 256;
@@ -596,12 +621,6 @@ FusedTile fused_tile(const fp64emu_layout_t& L) {
   const int64_t rounds = (t64 + kCUs - 1) / kCUs;
   if (nkt <= 8 ? rounds <= 4 : nkt <= 16 && rounds <= 2 && t64 * 10 >= rounds * kCUs * 9) return kFused64x64;
   return kFusedNone;
-}
-
-bool default_list(const int32_t* primes, int P) {
-  for (int t = 0; t < P; ++t)
-    if (primes[t] != kDefaultModuli[t]) return false;
-  return true;
 }
 
 // The layout of fp64emu_product, which leaves no stage for inspection: rows
@@ -3782,6 +3801,7 @@ int validate_primes(const int32_t* primes, int P) {
   if (P < 1) return fail(FP64EMU_EINVAL, "nprimes must be >= 1");
   if (P > kMaxP) return fail(FP64EMU_EINVAL, "too many primes");
   if (!primes) return fail(FP64EMU_EINVAL, "primes must not be NULL");
+  if (default_list(primes, P)) return FP64EMU_OK;
   for (int t = 0; t < P; ++t) {
     if (primes[t] < 2 || primes[t] > 256) return fail(FP64EMU_EINVAL, "moduli must be in [2, 256]");
     for (int u = 0; u < t; ++u)
@@ -3915,9 +3935,9 @@ int run(const Call& c) {
     }
     if (!fits) return fail(FP64EMU_EWORKSPACE, "workspace too small");
   }
-  const ModTables tab = make_tables(c.primes, c.P);
-  bool default_moduli = true;
-  for (int t = 0; t < c.P; ++t) default_moduli = default_moduli && c.primes[t] == kDefaultModuli[t];
+  ModTables own;
+  const ModTables& tab = call_tables(c.primes, c.P, &own);
+  const bool default_moduli = &tab != &own;
 
   char* ws = static_cast<char*>(c.ws);
   int16_t* sftA = reinterpret_cast<int16_t*>(ws + L.off_sftA);

@@ -35,13 +35,17 @@ at::Tensor workspace(const at::Tensor& like, size_t bytes) {
 // the largest of full/2, full/4, ... down to the minimum the library accepts
 // (it then runs the rows of A in as few chunks as fit).  Only batch-1 calls
 // with K <= 131071 have a smaller minimum; the others need the full size.
-at::Tensor workspace_fit(const at::Tensor& like, size_t full, size_t minimum) {
-  size_t want = full;
-  while (want > minimum) {
+template <typename Minimum>
+at::Tensor workspace_fit(const at::Tensor& like, size_t full, const Minimum& minimum_size) {
+  try {
+    return workspace(like, full);
+  } catch (const c10::OutOfMemoryError&) {
+  }
+  const size_t minimum = minimum_size();
+  for (size_t want = full / 2; want > minimum; want /= 2) {
     try {
       return workspace(like, want);
     } catch (const c10::OutOfMemoryError&) {
-      want /= 2;
     }
   }
   return workspace(like, minimum);
@@ -87,8 +91,9 @@ void product(at::Tensor& out, const at::Tensor& A, const at::Tensor& B, int64_t 
   p.exact = exact;
   p.bits = bits;
   p.use_corr = use_corr;
-  at::Tensor ws = workspace_fit(A, fp64emu_product_workspace(&p),
-                                fp64emu_workspace_size_min(batch, M, N, K, p.nprimes, use_corr));
+  at::Tensor ws = workspace_fit(A, fp64emu_product_workspace(&p), [&]() {
+    return fp64emu_workspace_size_min(batch, M, N, K, p.nprimes, use_corr);
+  });
   check_status(fp64emu_product(&p, ws.data_ptr(), (size_t)ws.numel(), current_stream(A)));
 }
 

@@ -56,9 +56,15 @@ def _tables(nprimes):
             torch.tensor(mu, dtype=torch.int64))
 
 
+@lru_cache(maxsize=1024)
+def _plan_config(K):
+    """plan_config, kept per depth: its sums of logarithms take 5 us."""
+    return plan_config(K)
+
+
 def _defaults(K, nprimes, corr):
     if nprimes is None or corr is None:
-        dp, dc = plan_config(K)
+        dp, dc = _plan_config(K)
         nprimes = dp if nprimes is None else nprimes
         corr = dc if corr is None else corr
     return nprimes, corr
