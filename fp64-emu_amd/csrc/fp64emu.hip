@@ -474,11 +474,16 @@ int choose_whole_k_split(int64_t items, int64_t nkt, int64_t group_slots, double
 
 bool whole_k_possible(int64_t K) { return K > kMaxKSingle && K <= kMaxSplit * (kMaxKSingle / kTileK * kTileK); }
 
+// How a call's work is laid out: as the staged entry points' (fp64emu_layout),
+// or one of fp64emu_product's forms, whole-K products (choose_whole_k_split)
+// and whole rounds (whole_rounds).
+enum class Form { kStaged, kWholeK, kWholeRounds };
+
 // nchunk_req > 1 (batch 1, not K-segmented): the planes of A and the output
 // planes hold one chunk of ceil(TM / nchunk_req) row tiles at a time.
-// whole_k: the whole-K form of a product deeper than one launch's bound.
 void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool corr,
-                 fp64emu_layout_t* L, int64_t nchunk_req = 1, bool whole_k = false) {
+                 fp64emu_layout_t* L, int64_t nchunk_req = 1, Form form = Form::kStaged) {
+  const bool whole_k = form == Form::kWholeK, rounds = form == Form::kWholeRounds;
   std::memset(L, 0, sizeof(*L));
   L->batch = batch; L->M = M; L->N = N; L->K = K;
   L->nprimes = P; L->use_corr = corr ? 1 : 0;
@@ -522,11 +527,12 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
                                      whole_k_small ? 0.37e-6 : 0.73e-6,
                                      (double)(batch * L->outplane_bytes) * (P + (corr ? 8 : 0)) / 4.0e12);
   }
+  if (rounds) L->ksplit = 1;
   // Under a K-split the two correction products run as two K-deep slots
   // (two int32 planes): a fused 2K-deep slot would make its groups twice as
   // long as every residue group (choose_ksplit already counts it as two).
-  if (L->ksplit > 1 && L->ncorr == 1) L->ncorr = 2;
-  if (!whole_k && use_split_streams(*L)) {
+  if ((L->ksplit > 1 || rounds) && L->ncorr == 1) L->ncorr = 2;
+  if (form == Form::kStaged && use_split_streams(*L)) {
     L->gemm_split = 1;
     L->ksplit = 2;
   }
@@ -569,8 +575,8 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
       if (L->nchunk == 1 && tiles <= 40) L->gemm_tile_rows = 128;
     }
   }
-  if (whole_k) L->gemm_tile_rows = L->gemm_tile_cols = whole_k_small ? 128 : 256;
-  L->gemm_run = use_slot_runs(*L) ? slot_run_length(*L) : 1;
+  if (form != Form::kStaged) L->gemm_tile_rows = L->gemm_tile_cols = whole_k_small ? 128 : 256;
+  L->gemm_run = !rounds && use_slot_runs(*L) ? slot_run_length(*L) : 1;
   // Plane rows the GEMM reads: 128-row (128-column) tiles read only the
   // first half of a 256-row plane tile past the last one holding data, so
   // the extraction skips the all-padding half there; a split stream's extra
@@ -630,17 +636,50 @@ FusedTile fused_tile(const fp64emu_layout_t& L) {
 // while its workspace stays below kWholeKBytes.
 constexpr size_t kWholeKBytes = (size_t)24 << 30;
 
+// Whole rounds: products of fewer 256 x 256 tiles than CUs whose tiles x slots
+// (the correction as two slots, each as deep as a residue's) come to whole
+// rounds of the chip run one slot per group without a K-split, every CU the
+// same k-steps.  The staged forms give such products 256 x 128 tiles, K-splits
+// or a double-length correction slot, for shapes whose tiles do not come out
+// even; here those cost operand traffic, split planes or a ragged last round.
+// Staged / whole rounds, whole calls, us (14 + correction: 16 slots a tile):
+//   1024^2 x 2560  (1 round)  107 /  95    2048^2 x 3000    (4)   300 /  281
+//   1024^2 x 16000 (1)        452 / 419    2048^2 x 8192    (4)   700 /  636
+//   1280 x 1536 x 3000 (1.9)  190 / 180    16 x 512^2 x 8192 (4) 1397 / 1323
+//   1024 x 2048 x 3000 (2)    187 / 163    16 x 256^2 x 32768 (1) 2632 / 2398
+//   1536 x 2048 x 8192 (3)    566 / 504    3000^2 x 8192    (9)  1249 / 1210
+// Shallow products need more rounds to gain: 1024^2 x 1536 (1) 65 / 77,
+// 1280 x 1536 x 2000 (1.9) 127 / 141, 2000^2 x 1000 (4) 132 / 135, 1024 x
+// 2048 x 2048 (2) 130 / 127, 2048^2 x 1500 (4) 172 / 168, 2000^3 (4) 217 / 208;
+// at 256 tiles and more the fused correction is balanced already (4096^2 x
+// 8192 1963 / 1992), and off whole rounds the staged forms stay (1024 x 1280 x
+// 3000, 1.25 rounds, 132 / 140).
+bool whole_rounds(const fp64emu_layout_t& L) {
+  if (L.deep || L.nchunk != 1) return false;
+  if (L.Np / kTileR >= 2 && L.N % kTileR != 0 && L.N % kTileR <= 128) return false;   // a mixed launch
+  const int64_t rows128 = round_up(std::max<int64_t>(L.M, 1), 128), cols128 = round_up(std::max<int64_t>(L.N, 1), 128);
+  if (rows128 * cols128 * 11 < L.Mp * L.Np * 10) return false;   // mostly padding at 256
+  const int64_t tiles = L.batch * (L.Mp / kTileR) * (L.Np / kTileR);
+  if (tiles >= kCUs) return false;
+  const int64_t units = tiles * (L.nprimes + (L.use_corr ? 2 : 0));
+  const int64_t n = (units + kCUs - 1) / kCUs, nkt = L.Kp / kTileK;
+  if (nkt >= 40) return units * 100 >= n * kCUs * 93;
+  return units * 100 >= n * kCUs * 99 && nkt >= (n >= 3 ? 24 : 32) && n >= 2;
+}
+
 void make_product_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool corr,
                          const int32_t* primes, FusedTile* fused, fp64emu_layout_t* L) {
-  bool whole = whole_k_possible(K);
-  make_layout(batch, M, N, K, P, corr, L, 1, whole);
-  if (whole && L->total > kWholeKBytes) {
-    whole = false;
-    make_layout(batch, M, N, K, P, corr, L);
+  *fused = kFusedNone;
+  make_layout(batch, M, N, K, P, corr, L, 1, whole_k_possible(K) ? Form::kWholeK : Form::kStaged);
+  if (whole_k_possible(K)) {
+    if (L->total > kWholeKBytes) make_layout(batch, M, N, K, P, corr, L);
+  } else {
+    if (default_list(primes, P)) *fused = fused_tile(*L);
+    if (*fused == kFusedNone && whole_rounds(*L))
+      make_layout(batch, M, N, K, P, corr, L, 1, Form::kWholeRounds);
   }
   L->ext_rowsA = round_up(std::max<int64_t>(M, 1), 64);
   L->ext_rowsB = round_up(std::max<int64_t>(N, 1), 64);
-  *fused = default_list(primes, P) ? fused_tile(*L) : kFusedNone;
   if (*fused != kFusedNone) L->total = L->off_res8;   // no residue or correction planes
 }
 

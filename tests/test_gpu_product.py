@@ -58,6 +58,19 @@ def test_unpadded_rows(dev, kind, batch, M, N, K, P, corr):
     _check(dev, kind, batch, M, N, K, P, corr)
 
 
+# Whole rounds: item streams (33 to 64 k-steps) and single items (more), the rounds not
+# quite whole, no correction (13 slots), members, ragged edges, both combines.
+@pytest.mark.parametrize("kind,batch,M,N,K,P,corr,exact", [
+    ("mm_nt", 1, 1000, 1024, 2600, 14, True, True),      # 1 round
+    ("mm", 1, 1279, 1500, 2561, 14, True, True),         # 1.9 rounds
+    ("bmm_nt", 19, 250, 256, 2700, 13, False, True),     # 247 of 256 units
+    ("bmm", 16, 256, 230, 4200, 14, True, False),        # past the streams' depth
+    ("mm", 1, 1792, 2000, 1537, 14, True, True),         # 3.5 rounds: staged
+])
+def test_whole_rounds(dev, kind, batch, M, N, K, P, corr, exact):
+    _check(dev, kind, batch, M, N, K, P, corr, exact)
+
+
 # Fused GEMM and reconstruction: each tile (32 x 32, 64 x 32, 64 x 64), edges inside and
 # at fragments and tiles, one k-step, depths that are not a multiple of the steps in
 # flight, members, both combines, 13 and 14 moduli, with and without the correction.
