@@ -724,6 +724,90 @@ __device__ __forceinline__ void row_pass(const double* __restrict__ x, int64_t c
 // flight), the four waves' sums meeting in LDS before the same fold.  A
 // block of kWaves waves holds kWaves / 4 such groups, or kWaves rows (one
 // per wave) otherwise.
+// Short rows (at most kShortRow elements) in numbers that fill the chip: a
+// wave takes kShortRows rows, all of two rows' loads in flight, and folds
+// their 64 lane sums together: each of the first three tree steps sends half
+// of the lane's rows across and keeps the other half (the same pairs added as
+// one row's tree adds them; a + b and b + a are the same bits), so the eight
+// rows cost 10 exchanges instead of 48, and their logarithms are taken side by
+// side.  Whole calls, a wave a row / eight: 64 x 256^3 (32768 rows) 110 / 105
+// us, 200 x 128^3 93 / 86, 100 x 200^3 157 / 148, 32 x 512^2 x 300 179 / 170;
+// even at 8192 rows (64 x 64^3) and slower at 512 elements (64 x 512^3 477 /
+// 482), whose loads alone fill the memory's queues.  Not for A's rows beside
+// a [K, N] operand's columns, whose groups bound that launch (200 x 100^3 77
+// / 82).
+constexpr int kShortRow = 320;
+constexpr int kShortRows = 8;
+constexpr int64_t kShortRowsFrom = 12288;
+
+template <int kU>
+__device__ __forceinline__ void short_row_sums(const double* const (&x)[2], int64_t K, int lane,
+                                               double (&t)[2], double (&m)[2]) {
+  double v[2][kU];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int u = 0; u < kU; ++u) v[h][u] = x[h] && 64 * u + lane < K ? x[h][64 * u + lane] : 0.0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    double ss[4] = {0.0, 0.0, 0.0, 0.0}, mx = 0.0;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      mx = fmax(mx, fabs(v[h][u]));
+      ss[u & 3] = fma(v[h][u], v[h][u], ss[u & 3]);
+    }
+    t[h] = (ss[0] + ss[2]) + (ss[1] + ss[3]);
+    m[h] = mx;
+  }
+}
+
+__device__ __forceinline__ void size_short_rows(int64_t row0, const double* __restrict__ A, int64_t rowsA,
+                                                const double* __restrict__ B, int64_t rows, int64_t K,
+                                                int bits, int16_t* __restrict__ sftA,
+                                                float* __restrict__ lgA, int16_t* __restrict__ sftB,
+                                                float* __restrict__ lgB) {
+  const int lane = threadIdx.x & 63;
+  double t[kShortRows], m[kShortRows];
+#pragma unroll
+  for (int r = 0; r < kShortRows; r += 2) {
+    const double* x[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t row = row0 + r + h;
+      x[h] = row >= rows ? nullptr : row < rowsA ? A + row * K : B + (row - rowsA) * K;
+    }
+    double t2[2], m2[2];
+    if (K <= 256) short_row_sums<4>(x, K, lane, t2, m2);
+    else short_row_sums<8>(x, K, lane, t2, m2);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      t[r + h] = t2[h];
+      m[r + h] = m2[h];
+    }
+  }
+  // Strides 32, 16, 8: lanes with the bit set keep the upper half of the rows.
+#pragma unroll
+  for (int n = kShortRows / 2, s = 32; n >= 1; n >>= 1, s >>= 1) {
+    const bool up = (lane & s) != 0;
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      const double ts = up ? t[i] : t[i + n], ms = up ? m[i] : m[i + n];
+      t[i] = (up ? t[i + n] : t[i]) + __shfl_xor(ts, s);
+      m[i] = fmax(up ? m[i + n] : m[i], __shfl_xor(ms, s));
+    }
+  }
+#pragma unroll
+  for (int s = 32 / kShortRows; s > 0; s >>= 1) {
+    t[0] = t[0] + __shfl_xor(t[0], s);
+    m[0] = fmax(m[0], __shfl_xor(m[0], s));
+  }
+  // Lane bits 5, 4, 3 are row bits 2, 1, 0.
+  const int64_t row = row0 + (lane >> 3);
+  if ((lane & 7) != 0 || row >= rows) return;
+  if (row < rowsA) row_stats_out(m[0], t[0], bits, &sftA[row], &lgA[row]);
+  else row_stats_out(m[0], t[0], bits, &sftB[row - rowsA], &lgB[row - rowsA]);
+}
+
 template <bool kGroup, int kWaves>
 __device__ __forceinline__ void size_rows_body(int64_t bid, const double* __restrict__ A, int64_t rowsA,
                                                const double* __restrict__ B, int64_t rows, int64_t K,
@@ -798,26 +882,49 @@ __device__ __forceinline__ void size_rows_body(int64_t bid, const double* __rest
   }
 }
 
-template <bool kGroup>
+// How rows are shared out: a wave each, a 256-thread group each, or eight
+// short ones a wave.
+enum RowMode { kRowWave, kRowGroup, kRowShort };
+
+template <RowMode kMode>
 __global__ void __launch_bounds__(kThreads)
 size_rows_kernel(const double* __restrict__ A, int64_t rowsA, const double* __restrict__ B,
                  int64_t rows, int64_t K, int bits, int16_t* __restrict__ sftA,
                  float* __restrict__ lgA, int16_t* __restrict__ sftB, float* __restrict__ lgB) {
-  size_rows_body<kGroup, kThreads / 64>(blockIdx.x, A, rowsA, B, rows, K, bits, sftA, lgA, sftB, lgB);
+  if constexpr (kMode == kRowShort)
+    size_short_rows(((int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6)) * kShortRows, A, rowsA, B, rows,
+                    K, bits, sftA, lgA, sftB, lgB);
+  else
+    size_rows_body<kMode == kRowGroup, kThreads / 64>(blockIdx.x, A, rowsA, B, rows, K, bits, sftA, lgA, sftB,
+                                                      lgB);
 }
 
 // A wave per row when the rows give the chip at least four waves per SIMD,
 // else a 256-thread group per row.
 constexpr int64_t kRowsGroupBelow = 4096;
+RowMode row_mode(int64_t rows, int64_t K) {
+  if (K <= kShortRow && rows >= kShortRowsFrom) return kRowShort;
+  return rows < kRowsGroupBelow ? kRowGroup : kRowWave;
+}
+
+int64_t row_groups(RowMode mode, int64_t rows) {
+  const int64_t per = mode == kRowGroup ? 1 : mode == kRowShort ? kRowsPerBlock * kShortRows : kRowsPerBlock;
+  return (rows + per - 1) / per;
+}
 
 void launch_size_rows(int64_t rows, hipStream_t s, const double* A, int64_t rowsA, const double* B,
                       int64_t K, int bits, int16_t* sftA, float* lgA, int16_t* sftB, float* lgB) {
-  if (rows < kRowsGroupBelow)
-    hipLaunchKernelGGL(size_rows_kernel<true>, dim3((unsigned)rows), dim3(kThreads), 0, s, A, rowsA,
-                       B, rows, K, bits, sftA, lgA, sftB, lgB);
+  const RowMode mode = row_mode(rows, K);
+  const dim3 grid((unsigned)row_groups(mode, rows)), block(kThreads);
+  if (mode == kRowGroup)
+    hipLaunchKernelGGL(size_rows_kernel<kRowGroup>, grid, block, 0, s, A, rowsA, B, rows, K, bits, sftA, lgA,
+                       sftB, lgB);
+  else if (mode == kRowShort)
+    hipLaunchKernelGGL(size_rows_kernel<kRowShort>, grid, block, 0, s, A, rowsA, B, rows, K, bits, sftA, lgA,
+                       sftB, lgB);
   else
-    hipLaunchKernelGGL(size_rows_kernel<false>, dim3((unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock)),
-                       dim3(kThreads), 0, s, A, rowsA, B, rows, K, bits, sftA, lgA, sftB, lgB);
+    hipLaunchKernelGGL(size_rows_kernel<kRowWave>, grid, block, 0, s, A, rowsA, B, rows, K, bits, sftA, lgA,
+                       sftB, lgB);
 }
 
 // The sizing of A's rows and of the [K, N] operand's columns in one launch
@@ -4042,7 +4149,7 @@ int run(const Call& c) {
     // kSizeThreads wide.)
     const bool group = MF < kRowsGroupBelow;
     const int64_t sizing =
-        !c.b_kn ? (MF + NF < kRowsGroupBelow ? MF + NF : (MF + NF + kRowsPerBlock - 1) / kRowsPerBlock)
+        !c.b_kn ? row_groups(row_mode(MF + NF, c.K), MF + NF)
         : kslab <= kFusedSlabRows
             ? ((group ? (MF + kSizeThreads / 256 - 1) / (kSizeThreads / 256)
                       : (MF + kSizeThreads / 64 - 1) / (kSizeThreads / 64)) +

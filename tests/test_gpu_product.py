@@ -100,3 +100,31 @@ def test_fused_zero_and_nonfinite(dev):
         ref, _, _ = capi.run("mm", A, B, O.PRIMES[:14])
         torch.cuda.synchronize()
         assert bits_equal(got.cpu().numpy(), ref.cpu().numpy())
+
+
+# Sizing of short rows, eight a wave: rows that end inside a wave's eight and a group's
+# 32, one to 320 elements, rows of every scale, an all-zero and an infinite row.
+@pytest.mark.parametrize("batch,M,N,K", [(97, 64, 63, 1), (64, 100, 97, 65), (49, 130, 127, 256), (41, 150, 151, 257),
+                                         (31, 200, 203, 320)])
+def test_short_row_sizing(dev, batch, M, N, K):
+    import numpy as np
+    from parity_util import oracle_sizing
+    print(f"case short rows bmm b={batch} {M}x{N}x{K}", flush=True)
+    g = torch.Generator().manual_seed(K)
+    A = torch.randn((batch, M, K), dtype=torch.float64, generator=g)
+    B = torch.randn((batch, N, K), dtype=torch.float64, generator=g)
+    for X in (A, B):
+        X *= torch.pow(2.0, torch.randint(-60, 61, X.shape[:2] + (1,), generator=g).double())
+    A[3, 5] = 0.0
+    B[7, 11, 0] = float("inf")
+    assert batch * (M + N) >= 12288
+    _, ws, lay = capi.run("bmm", A.to(dev), B.to(dev), O.PRIMES[:14])
+    torch.cuda.synchronize()
+    gsA, gsB, glA, glB, gbe = capi.sizing(ws[:lay.off_planesA].cpu().numpy(), lay)
+    be, sA, sB, lA, lB = oracle_sizing(A.numpy(), B.numpy(), False, O.PRIMES[:14], 53)
+    assert gbe == be and np.array_equal(gsA, sA) and np.array_equal(gsB, sB)
+    for got, want in ((glA, lA), (glB, lB)):   # float log2-norms: an ulp, rarely (libm's log2)
+        off = got != want
+        assert off.mean() < 1e-3
+        gi, wi = got[off].view(np.int32).astype(np.int64), want[off].view(np.int32).astype(np.int64)
+        assert np.all(np.abs(gi - wi) <= 1)
