@@ -3585,8 +3585,15 @@ fused_kernel(FusedArgs g) {
         acc[x][y] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[x], B[y], acc[x][y], 0, 0, 0);
       }
   };
+  // A slot's first k-steps, no more than it has: every load takes the CU's
+  // one vector memory path 16 cycles (redundant ones at the ends cost 64^3
+  // 14.2 us instead of 13.2, 64 x 256^3 104.8 instead of 100.6).
+  auto prefetch = [&](const int t) {
 #pragma unroll
-  for (int d = 0; d < kD; ++d) load(FA[d], FB[d], min(t0, kP), min(d, n - 1));
+    for (int d = 0; d < kD; ++d)
+      if (d < n) load(FA[d], FB[d], t, d);
+  };
+  prefetch(t0);
 
   const int be = g.bits_eff[0], grow = g.bits_eff[1];
   const int64_t om0 = (int64_t)mt * (16 * kTM) + 4 * (lane >> 4) + 2 * sub, on0 = (int64_t)nt * (16 * kTN) + (lane & 15);
@@ -3600,21 +3607,23 @@ fused_kernel(FusedArgs g) {
     const double ip = kDefaultTab.invp[tc];
     const int negp = -kDefaultTab.p[tc];
     int k = 0;
-    for (; k + kD < n; k += kD) {
+    for (; k + 2 * kD <= n; k += kD) {
 #pragma unroll
       for (int d = 0; d < kD; ++d) {
         mma(FA[d], FB[d]);
-        load(FA[d], FB[d], t, min(k + d + kD, n - 1));
+        load(FA[d], FB[d], t, k + d + kD);
       }
     }
-    // The last 1 .. kD k-steps; then the next slot's first ones.
+    // The last 1 .. 2 kD - 1 k-steps; then the next slot's first ones.
 #pragma unroll
-    for (int d = 0; d < kD; ++d)
+    for (int d = 0; d < kD; ++d) {
       if (k + d < n) mma(FA[d], FB[d]);
-    if (t + tstep < kP && !corr_wave) {
-#pragma unroll
-      for (int d = 0; d < kD; ++d) load(FA[d], FB[d], t + tstep, min(d, n - 1));
+      if (k + d + kD < n) load(FA[d], FB[d], t, k + d + kD);
     }
+#pragma unroll
+    for (int d = 0; d + 1 < kD; ++d)
+      if (k + d + kD < n) mma(FA[d], FB[d]);
+    if (t + tstep < kP && !corr_wave) prefetch(t + tstep);
     if (corr_wave) {
 #pragma unroll
       for (int x = 0; x < kTM; ++x)
