@@ -17,7 +17,7 @@
 namespace {
 
 constexpr int64_t kMaxKSingle = 131071;
-constexpr int64_t kMaxKDeep = (int64_t)128 * 65536;   // K-segmented bound (mm, bmm)
+constexpr int64_t kMaxKDeep = (int64_t)128 * 65536;   // the deep bound (mm, bmm)
 
 void check_status(int st) { TORCH_CHECK(st == FP64EMU_OK, fp64emu_last_error()); }
 
@@ -111,7 +111,7 @@ void fp64_emu_mm(at::Tensor& out, const at::Tensor& A, const at::Tensor& B,
   const int64_t M = A.size(0), K = A.size(1), N = B.size(0);
   TORCH_CHECK(B.size(1) == K, "expect B as [N, K]");
   check_out(out, A, {M, N}, "out f64 [M,N]");
-  // Deeper than 131071 runs K-segmented, to 128 segments of 65536.
+  // Past one launch's 131071, whole or K-segmented: to 128 segments of 65536.
   TORCH_CHECK(K <= kMaxKDeep, "K bound: 128 segments of 65536");
   product(out, A, B, 1, M, N, K, false, primes_cpu, exact, bits, use_corr);
 }
