@@ -3462,7 +3462,9 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
 // (fused_tile): a group takes one output tile of 16 kTM x 16 kTN through every
 // slot and reconstructs it, so that no residue or correction plane is written
 // and read back (36 bytes an output at 14 moduli against the 8 of the result)
-// and the call is one launch shorter.
+// and the call is one launch shorter.  Whole calls, staged / fused: 64^3 22.4 /
+// 19.9 us, 333 x 501 x 777 38.0 / 35.3, 1024^3 64.8 / 50.0, 64 x 256^3 140.7 /
+// 116.7 (when it came in; the steps since changed the rest of these calls too).
 //
 // The eight waves split the slots, not the tile: one takes the correction (two
 // residue slots' worth of k-steps) and the others two residue slots each, at
