@@ -58,13 +58,14 @@ def _tables(nprimes):
 
 @lru_cache(maxsize=1024)
 def _plan_config(K):
-    """plan_config, kept per depth: its sums of logarithms take 5 us."""
+    """plan_config, kept per depth: its sums of logarithms take 5 us.  Only for
+    a plain int: a traced call's symbolic size has no hash."""
     return plan_config(K)
 
 
 def _defaults(K, nprimes, corr):
     if nprimes is None or corr is None:
-        dp, dc = _plan_config(K)
+        dp, dc = _plan_config(K) if type(K) is int else plan_config(K)
         nprimes = dp if nprimes is None else nprimes
         corr = dc if corr is None else corr
     return nprimes, corr
