@@ -608,15 +608,21 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
 //   1500^2 x 256    58.0  50.1  51.0  58.8    32 x 512^3       267   315   290   301
 //   1500^2 x 700    83.4  97.8  88.0  90.3    64 x 512^2 x 128 263   240   201   249
 enum FusedTile { kFusedNone, kFused32x32, kFused64x32, kFused64x64 };
+constexpr int kFusedThreads = 512;
 
-FusedTile fused_tile(const fp64emu_layout_t& L) {
+int64_t fused_rows(FusedTile t) { return t == kFused32x32 ? 32 : 64; }
+int64_t fused_cols(FusedTile t) { return t == kFused64x64 ? 64 : 32; }
+int64_t fused_groups(const fp64emu_layout_t& L, FusedTile t) {
+  return L.batch * ((L.M + fused_rows(t) - 1) / fused_rows(t)) * ((L.N + fused_cols(t) - 1) / fused_cols(t));
+}
+
+FusedTile fused_tile_choice(const fp64emu_layout_t& L) {
   // Compiled for the planner's modulus counts at these depths; the fused
   // correction's int32 bound; 32-bit offsets inside a member's planes.
   if (L.deep || L.nchunk != 1 || (L.nprimes != 13 && L.nprimes != 14)) return kFusedNone;
   if (L.memberA_bytes > 0xFFFFFFFFll || L.memberB_bytes > 0xFFFFFFFFll || L.K > kMaxKFusedCorr) return kFusedNone;
   const int64_t nkt = L.Kp / kTileK;
-  auto tiles = [&](int64_t r, int64_t c) { return L.batch * ((L.M + r - 1) / r) * ((L.N + c - 1) / c); };
-  const int64_t t32 = tiles(32, 32), t64 = tiles(64, 64);
+  const int64_t t32 = fused_groups(L, kFused32x32), t64 = fused_groups(L, kFused64x64);
   if (t32 <= kCUs)   // under a tile per CU; few and deep, the staged K-split spreads them wider
     return nkt <= std::max<int64_t>(8, t32 / 4) ? kFused32x32 : kFusedNone;
   if (t64 <= kCUs) {   // one round of the large tile, or (few of those) up to two of the small
@@ -627,6 +633,14 @@ FusedTile fused_tile(const fp64emu_layout_t& L) {
   const int64_t rounds = (t64 + kCUs - 1) / kCUs;
   if (nkt <= 8 ? rounds <= 4 : nkt <= 16 && rounds <= 2 && t64 * 10 >= rounds * kCUs * 9) return kFused64x64;
   return kFusedNone;
+}
+
+// The fused launch of a product, or none where its groups pass the 2^32 - 1
+// work-items of a dispatch: the staged form's launches (of fewer work-items an
+// output where rows end early in their tiles) may still hold such a product.
+FusedTile fused_tile(const fp64emu_layout_t& L) {
+  const FusedTile t = fused_tile_choice(L);
+  return t != kFusedNone && fused_groups(L, t) > (int64_t)0xFFFFFFFFu / kFusedThreads ? kFusedNone : t;
 }
 
 // The layout of fp64emu_product, which leaves no stage for inspection: rows
@@ -3514,7 +3528,6 @@ struct FusedArgs {
   FastDiv div_grp;     // by 8 TN (8 row tiles, every column tile)
 };
 
-constexpr int kFusedThreads = 512;
 constexpr int kFusedWaves = kFusedThreads / 64;
 
 // kD: k-steps in flight per wave; kWavesPerSimd: the register budget.
@@ -4168,9 +4181,8 @@ int run(const Call& c) {
             : (group ? MF : (MF + kRowsPerBlock - 1) / kRowsPerBlock) + (NF + kThreads - 1) / kThreads * nslab;
     const int64_t extraction = c.batch * (L.ext_rowsA / 64 + L.ext_rowsB / 64) * (L.Kp / kTileK);
     const int64_t recon = c.batch * ((std::min<int64_t>(L.chunk_rows, c.M) + 15) / 16) * ((c.N + 63) / 64);
-    // (Fused groups, twice kThreads wide, of at least 32 x 32 outputs.)
-    const int64_t tiles = fused == kFusedNone ? 0 : 2 * c.batch * ((c.M + 31) / 32) * ((c.N + 31) / 32);
-    for (int64_t gsz : {sizing, extraction, ga.total, recon, tiles})
+    // (A fused launch is in bounds by choice: fused_tile.)
+    for (int64_t gsz : {sizing, extraction, ga.total, recon})
       if (gsz > limit) return fail(FP64EMU_EINVAL, "problem too large for one launch");
   }
 
@@ -4270,7 +4282,7 @@ int run(const Call& c) {
         if (int st = check_hip(hipEventRecord(c.ev[1], s), "hipEventRecord")) return st;
       }
       if (fused != kFusedNone) {
-        const int64_t rows = fused == kFused32x32 ? 32 : 64, cols = fused == kFused64x64 ? 64 : 32;
+        const int64_t rows = fused_rows(fused), cols = fused_cols(fused);
         FusedArgs fa;
         fa.A = planesA; fa.B = planesB; fa.out = c.out;
         fa.sftA = sftA; fa.sftB = sftB; fa.bits_eff = bits_eff;

@@ -130,6 +130,14 @@ def workspace_size_min(batch, M, N, K, nprimes, use_corr):
     return lib().fp64emu_workspace_size_min(batch, M, N, K, nprimes, int(bool(use_corr)))
 
 
+def product_workspace(batch, M, N, K, primes, use_corr=True, nt=False):
+    """fp64emu_product_workspace of a product of these sizes and moduli."""
+    primes = np.ascontiguousarray(np.asarray(primes, dtype=np.int32))
+    p = Product(None, None, None, batch, M, N, K, int(bool(nt)), primes.ctypes.data, primes.size, 1, 53,
+                int(bool(use_corr)))
+    return lib().fp64emu_product_workspace(ctypes.byref(p))
+
+
 def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
