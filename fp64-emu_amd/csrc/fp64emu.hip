@@ -472,6 +472,12 @@ int choose_whole_k_split(int64_t items, int64_t nkt, int64_t group_slots, double
   return best;
 }
 
+// Planes of 128-row tiles: whole-K products on 128 x 128 tiles, whose planes
+// are most of the workspace (17 bytes an element at 15 moduli) and would be
+// half padding in tiles of 256 rows.  (No staged layout past K = 131071 is
+// whole: L.deep.)
+bool half_planes(const fp64emu_layout_t& L) { return !L.deep && L.K > kMaxKSingle && L.gemm_tile_rows == 128; }
+
 bool whole_k_possible(int64_t K) { return K > kMaxKSingle && K <= kMaxSplit * (kMaxKSingle / kTileK * kTileK); }
 
 // How a call's work is laid out: as the staged entry points' (fp64emu_layout),
@@ -500,11 +506,18 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
   L->Mp = round_up(std::max<int64_t>(M, 1), kTileR);
   L->Np = round_up(std::max<int64_t>(N, 1), kTileR);
   L->Kp = round_up(L->kseg, kTileK);
-  const int64_t TM = L->Mp / kTileR;
+  // Whole-K products take 128 x 128 tiles (two groups per CU), on planes of
+  // 128-row tiles (half_planes), where those cut the padded work by more than
+  // 10%.
+  const int64_t rows128 = round_up(std::max<int64_t>(M, 1), 128), cols128 = round_up(std::max<int64_t>(N, 1), 128);
+  const bool whole_k_small = whole_k && rows128 * cols128 * 11 < L->Mp * L->Np * 10;
+  if (whole_k_small) { L->Mp = rows128; L->Np = cols128; }
+  const int64_t tile_rows = whole_k_small ? 128 : kTileR;
+  const int64_t TM = L->Mp / tile_rows;
   int64_t ctiles = TM;
   if (nchunk_req > 1 && batch == 1 && !L->deep) ctiles = (TM + nchunk_req - 1) / nchunk_req;
   L->nchunk = (int)((TM + ctiles - 1) / ctiles);
-  L->chunk_rows = ctiles * kTileR;
+  L->chunk_rows = ctiles * tile_rows;
   L->planeA_bytes = L->chunk_rows * L->Kp;
   L->planeB_bytes = L->Np * L->Kp;
   const int nplanes = P + (corr ? 2 : 0);   // the correction plane is 2*Kp deep
@@ -515,13 +528,8 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
   // and int64 correction sums across the segments.)
   L->ksplit = choose_ksplit(batch, ctiles * (L->Np / kTileR), L->Kp / kTileK, P, L->ncorr,
                             batch * L->outplane_bytes, batch * (L->memberA_bytes + L->memberB_bytes));
-  bool whole_k_small = false;
   if (whole_k) {
-    // 128 x 128 tiles (two groups per CU) where they cut the padded work by
-    // more than 10%.
-    const int64_t rows128 = round_up(std::max<int64_t>(M, 1), 128), cols128 = round_up(std::max<int64_t>(N, 1), 128);
-    whole_k_small = rows128 * cols128 * 11 < L->Mp * L->Np * 10;
-    const int64_t tiles = whole_k_small ? rows128 / 128 * (cols128 / 128) : TM * (L->Np / kTileR);
+    const int64_t tiles = TM * (L->Np / tile_rows);
     const int slots = P + (corr ? 2 : 0);
     L->ksplit = choose_whole_k_split(batch * tiles * slots, L->Kp / kTileK, whole_k_small ? 2 * kCUs : kCUs,
                                      whole_k_small ? 0.37e-6 : 0.73e-6,
@@ -555,7 +563,6 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
   L->gemm_tile_cols = (!L->gemm_split && use_narrow_gemm(*L)) ? 128 : 256;
   // 128 x 128 tiles where 128-row tiles also cut the padded work by > 10%
   // (M <= 128: half): two groups per CU, a quarter of the 256 x 256 work.
-  const int64_t rows128 = (std::max<int64_t>(M, 1) + 127) / 128 * 128;
   L->gemm_tile_rows = (L->gemm_tile_cols == 128 && L->nchunk == 1 && rows128 * 11 < L->Mp * 10)
                           ? 128 : 256;
   // Shallow products (at most kRunMaxSteps k-steps, no K-split, two moduli or
@@ -646,9 +653,17 @@ FusedTile fused_tile(const fp64emu_layout_t& L) {
 // The layout of fp64emu_product, which leaves no stage for inspection: rows
 // past the operands' last 64-row group are never written (a GEMM output
 // depends on its own row and column alone, and the reconstruction reads the
-// valid ones), and a product past one launch's depth runs whole (whole_k)
-// while its workspace stays below kWholeKBytes.
-constexpr size_t kWholeKBytes = (size_t)24 << 30;
+// valid ones), and a product past one launch's depth runs whole
+// (Form::kWholeK) while its workspace stays within
+// FP64EMU_WHOLE_K_BYTES and kWholeKTimes times the operands' bytes or the
+// segmented form's workspace.  Deeper, few rows are mostly padding: 1 x 1 x
+// 2000000 would take 8.7 GB for 32 MB of operands (segmented 0.6).
+constexpr int kWholeKTimes = 5;
+
+bool whole_k_fits(const fp64emu_layout_t& whole, const fp64emu_layout_t& segmented) {
+  const size_t operands = sizeof(double) * (size_t)(whole.batch * (whole.M + whole.N) * whole.K);
+  return whole.total <= std::min<size_t>(FP64EMU_WHOLE_K_BYTES, kWholeKTimes * std::max(operands, segmented.total));
+}
 
 // Whole rounds: products of fewer 256 x 256 tiles than CUs whose tiles x slots
 // (the correction as two slots, each as deep as a residue's) come to whole
@@ -684,9 +699,11 @@ bool whole_rounds(const fp64emu_layout_t& L) {
 void make_product_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool corr,
                          const int32_t* primes, FusedTile* fused, fp64emu_layout_t* L) {
   *fused = kFusedNone;
-  make_layout(batch, M, N, K, P, corr, L, 1, whole_k_possible(K) ? Form::kWholeK : Form::kStaged);
+  make_layout(batch, M, N, K, P, corr, L);
   if (whole_k_possible(K)) {
-    if (L->total > kWholeKBytes) make_layout(batch, M, N, K, P, corr, L);
+    fp64emu_layout_t whole;
+    make_layout(batch, M, N, K, P, corr, &whole, 1, Form::kWholeK);
+    if (whole_k_fits(whole, *L)) *L = whole;
   } else {
     if (default_list(primes, P)) *fused = fused_tile(*L);
     if (*fused == kFusedNone && whole_rounds(*L))
@@ -1342,10 +1359,12 @@ constexpr int64_t kSmallExtractGroups = 384;
 // kDefault: the modulus list is a prefix of the default one, whose constants
 // the plane loop takes at compile time (no scalar load and wait per plane,
 // which dominated small launches); otherwise the tables of the arguments.
-template <bool kDefault, int kEl>
+// kPlaneRows: rows of a plane tile (half_planes).
+template <bool kDefault, int kEl, int kPlaneRows = kTileR>
 __global__ void __launch_bounds__(kThreads)
 extract_kernel(ExtractArgs<!kDefault> a) {
   constexpr int kW = kEl / 4;   // packed residue words per lane and plane
+  constexpr int kPlaneTile = kPlaneRows * kTileK;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // The width pick, when this launch takes it: every wave reaches the
   // block's barrier before any returns.  Small launches (kEl = 4) read the
@@ -1419,11 +1438,12 @@ extract_kernel(ExtractArgs<!kDefault> a) {
   // operand) only stores zeros: no loads and no residue arithmetic.
   const int P = a.P;
   const int64_t nkt = a.nkt;
-  const int64_t rt = rblk >> 4, fr = rblk & 15;
+  constexpr int kTileShift = kPlaneRows == 128 ? 3 : 4;   // log2 of a plane tile's 16-row blocks
+  const int64_t rt = rblk >> kTileShift, fr = rblk & ((1 << kTileShift) - 1);
   const int64_t plane = isA ? a.planeA : a.planeB;
   int8_t* base = (isA ? a.planesA : a.planesB) + b * (isA ? a.memberA : a.memberB);
   const int in_frag = kEl == 16 ? lane * 16 : wave * 256 + (lane & 15) * 16 + (lane >> 4) * 4;
-  const int64_t off = (rt * nkt + kt) * kTileBytes + fr * kFragBytes + in_frag;
+  const int64_t off = (rt * nkt + kt) * kPlaneTile + fr * kFragBytes + in_frag;
   typedef std::conditional_t<kEl == 16, v4i, int> Words;
   auto store_words = [&](int8_t* at, const uint32_t (&w)[kW]) {
     if constexpr (kEl == 16) *reinterpret_cast<v4i*>(at) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
@@ -1455,9 +1475,9 @@ extract_kernel(ExtractArgs<!kDefault> a) {
     for (int pi = 0; pi < P; ++pi) *reinterpret_cast<Words*>(base + pi * plane + off) = z;
     if (a.use_corr) {
       int8_t* cb = base + (int64_t)P * plane;
-      const int64_t o1 = (rt * 2 * nkt + kt) * kTileBytes + fr * kFragBytes + in_frag;
+      const int64_t o1 = (rt * 2 * nkt + kt) * kPlaneTile + fr * kFragBytes + in_frag;
       *reinterpret_cast<Words*>(cb + o1) = z;
-      *reinterpret_cast<Words*>(cb + o1 + nkt * kTileBytes) = z;
+      *reinterpret_cast<Words*>(cb + o1 + nkt * kPlaneTile) = z;
     }
     return;
   }
@@ -1561,8 +1581,8 @@ extract_kernel(ExtractArgs<!kDefault> a) {
   if (a.use_corr) {
     // Correction plane: row tile stride 2*nkt tiles; A = [hi | q], B = [q | hi].
     int8_t* cb = base + (int64_t)P * plane;
-    const int64_t o1 = (rt * 2 * nkt + kt) * kTileBytes + fr * kFragBytes + in_frag;
-    const int64_t o2 = o1 + nkt * kTileBytes;
+    const int64_t o1 = (rt * 2 * nkt + kt) * kPlaneTile + fr * kFragBytes + in_frag;
+    const int64_t o2 = o1 + nkt * kPlaneTile;
     store_words(cb + o1, isA ? hw : qw);
     store_words(cb + o2, isA ? qw : hw);
   }
@@ -1841,7 +1861,7 @@ __device__ __forceinline__ void store_residue_block(const v4i (&acc)[kWM][kWN], 
 // single LDS object).  kStream: an item stream; with kSplitS, a split stream,
 // with kXc > 0 computing the kXc extra columns beside the last wide tiles.
 template <bool kDeep, int kWM, int kWN, bool kRun = false, bool kStream = false,
-          bool kSplitS = false, int kXc = 0>
+          bool kSplitS = false, int kXc = 0, int kPlaneRows = kTileR>
 __device__ __forceinline__ void modgemm_tile(const GemmArgs& g, int8_t* lds, const GemmItem it) {
   using Sh = GemmShape<kWM, kWN>;
   constexpr int kSB = Sh::kSB, kDma = Sh::kDma, kHB = Sh::kHB;
@@ -1868,15 +1888,19 @@ __device__ __forceinline__ void modgemm_tile(const GemmArgs& g, int8_t* lds, con
   const int kt0 = ((is_corr && g.ncorr == 2) ? slot * g.nkt : 0) + kbeg;
 
   // A 128-row (or 128-column) tile is one half (8 fragments) of a 256-row
-  // plane tile.
-  const int mrt = kWM == 8 ? mt : mt >> 1;
-  const int mhalf = kWM == 8 ? 0 : mt & 1;
+  // plane tile, or a plane tile of its own (kPlaneRows = 128).
+  static_assert(kPlaneRows == kTileR || (kWM == 4 && kWN == 4 && !kDeep && !kRun && !kStream),
+                "planes of 128-row tiles: 128 x 128 GEMM tiles");
+  constexpr int kPlaneTile = kPlaneRows * kTileK;
+  constexpr bool kHalves = kPlaneRows == kTileR;
+  const int mrt = kWM == 8 || !kHalves ? mt : mt >> 1;
+  const int mhalf = kWM == 8 || !kHalves ? 0 : mt & 1;
   const int8_t* At = g.A + b * g.memberA + (int64_t)plane * g.planeA +
-                     ((int64_t)mrt * rstride + kt0) * kTileBytes + mhalf * kAB;
-  const int nrt = kWN == 8 ? nt : nt >> 1;
-  const int nhalf = kWN == 8 ? 0 : nt & 1;
+                     ((int64_t)mrt * rstride + kt0) * kPlaneTile + mhalf * kAB;
+  const int nrt = kWN == 8 || !kHalves ? nt : nt >> 1;
+  const int nhalf = kWN == 8 || !kHalves ? 0 : nt & 1;
   const int8_t* Bt = g.B + b * g.memberB + (int64_t)plane * g.planeB +
-                     ((int64_t)nrt * rstride + kt0) * kTileBytes + nhalf * Sh::kBBytes;
+                     ((int64_t)nrt * rstride + kt0) * kPlaneTile + nhalf * Sh::kBBytes;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1939,10 +1963,10 @@ __device__ __forceinline__ void modgemm_tile(const GemmArgs& g, int8_t* lds, con
     }                                                                                       \
   } while (0)
 #define FP64EMU_COPY_A(kt, j)                                                               \
-  copy_lds16<(j) * 1024>((kRun || kStream ? cpA : At + (int64_t)(kt) * kTileBytes) + goff,   \
+  copy_lds16<(j) * 1024>((kRun || kStream ? cpA : At + (int64_t)(kt) * kPlaneTile) + goff,   \
                          (lds_i8*)(lds + FP64EMU_SLOT(kt) * kSB + wave * (kWM / 2) * 1024))
 #define FP64EMU_COPY_B(kt, j)                                                               \
-  copy_lds16<(j) * 1024>((kRun || kStream ? cpB : Bt + (int64_t)(kt) * kTileBytes) + goffB,  \
+  copy_lds16<(j) * 1024>((kRun || kStream ? cpB : Bt + (int64_t)(kt) * kPlaneTile) + goffB,  \
                          (lds_i8*)(lds + FP64EMU_SLOT(kt) * kSB + kAB + wave * (kWN / 2) * 1024))
 #define FP64EMU_ISSUE(kt)                                                              \
   do {                                                                                 \
@@ -2686,7 +2710,7 @@ __device__ __forceinline__ void modgemm_tile(const GemmArgs& g, int8_t* lds, con
   }
 }
 
-template <bool kDeep, int kWM, int kWN, bool kRun = false, bool kStream = false>
+template <bool kDeep, int kWM, int kWN, bool kRun = false, bool kStream = false, int kPlaneRows = kTileR>
 __global__ void __launch_bounds__(kThreads, (kWM == 8 && kWN == 8) ? 1 : 2)
 modgemm_kernel(GemmArgs g) {
   static_assert(!(kRun || kStream) || (kWM == 8 && kWN == 8 && !kDeep),
@@ -2704,7 +2728,7 @@ modgemm_kernel(GemmArgs g) {
       return;
     }
   }
-  modgemm_tile<kDeep, kWM, kWN>(g, lds, it);
+  modgemm_tile<kDeep, kWM, kWN, false, false, false, 0, kPlaneRows>(g, lds, it);
 }
 
 // 256-column tiles, except that the last tile column holds at most 128
@@ -4134,6 +4158,7 @@ int run(const Call& c) {
   // their column tiles past N hold only padding and are not launched.
   const bool narrow = L.gemm_tile_cols == 128;
   const bool small = narrow && L.gemm_tile_rows == 128;
+  const bool half = half_planes(L);   // small, and a whole-K product
   // Wide tiles whose last tile column holds at most 128 columns of N: that
   // column runs 128-column tiles in the same launch.
   const bool mixed = use_mixed_tiles(L);
@@ -4223,7 +4248,7 @@ int run(const Call& c) {
   }
   const float log2M = std::min(tab.log2M, 126.0f);
   const int64_t groups64 = c.batch * (L.ext_rowsA / 64 + L.ext_rowsB / 64) * (L.Kp / kTileK);
-  const int64_t ext_rows = default_moduli && groups64 <= kSmallExtractGroups ? 16 : 64;   // rows of an extraction group
+  const int64_t ext_rows = default_moduli && !half && groups64 <= kSmallExtractGroups ? 16 : 64;   // rows of an extraction group
   const int64_t ext_groups = groups64 * (64 / ext_rows);
   const bool pick_in_extract = L.nchunk == 1 && L.nseg == 1 && MF + NF <= kPickInExtractMax &&
                                (MF + NF) * (int64_t)sizeof(float) * ext_groups <= kPickInExtractBytes;
@@ -4268,7 +4293,9 @@ int run(const Call& c) {
       if (default_moduli) {
         ExtractArgs<false> ed;
         static_cast<ExtractCore&>(ed) = ea;
-        if (ext_rows == 16)
+        if (half)
+          hipLaunchKernelGGL((extract_kernel<true, 16, 128>), dim3((unsigned)wg), dim3(kThreads), 0, s, ed);
+        else if (ext_rows == 16)
           hipLaunchKernelGGL((extract_kernel<true, 4>), dim3((unsigned)wg), dim3(kThreads), 0, s, ed);
         else
           hipLaunchKernelGGL((extract_kernel<true, 16>), dim3((unsigned)wg), dim3(kThreads), 0, s, ed);
@@ -4276,7 +4303,10 @@ int run(const Call& c) {
         ExtractArgs<true> eg;
         static_cast<ExtractCore&>(eg) = ea;
         eg.tab = tab;
-        hipLaunchKernelGGL((extract_kernel<false, 16>), dim3((unsigned)wg), dim3(kThreads), 0, s, eg);
+        if (half)
+          hipLaunchKernelGGL((extract_kernel<false, 16, 128>), dim3((unsigned)wg), dim3(kThreads), 0, s, eg);
+        else
+          hipLaunchKernelGGL((extract_kernel<false, 16>), dim3((unsigned)wg), dim3(kThreads), 0, s, eg);
       }
       if (c.ev) {
         if (int st = check_hip(hipEventRecord(c.ev[1], s), "hipEventRecord")) return st;
@@ -4310,6 +4340,9 @@ int run(const Call& c) {
         hipLaunchKernelGGL(modgemm_split_kernel, dim3(kCUs), dim3(kThreads), 0, s, ga);
       else if (ga.run > 1)   // 256 x 256 tiles only (use_slot_runs)
         hipLaunchKernelGGL((modgemm_kernel<false, 8, 8, true>), dim3((unsigned)ga.total), dim3(kThreads), 0, s, ga);
+      else if (half)
+        hipLaunchKernelGGL((modgemm_kernel<false, 4, 4, false, false, 128>), dim3((unsigned)ga.total),
+                           dim3(kThreads), 0, s, ga);
       else if (small)
         hipLaunchKernelGGL((modgemm_kernel<false, 4, 4>), dim3((unsigned)ga.total), dim3(kThreads), 0, s, ga);
       else if (narrow)

@@ -176,7 +176,11 @@ typedef struct {
 
 /* Workspace of fp64emu_product (out, A and B may be NULL here).  On a shorter
  * one the call runs as the entry points above would, down to
- * fp64emu_workspace_size_min(). */
+ * fp64emu_workspace_size_min().  Products of K > 131071 ask for more than
+ * fp64emu_workspace_size() where their planes over the whole depth stay within
+ * FP64EMU_WHOLE_K_BYTES and within five times the operands' bytes or that
+ * size, whichever is larger; otherwise they run K-segmented in that size. */
+#define FP64EMU_WHOLE_K_BYTES (24ull << 30)
 size_t fp64emu_product_workspace(const fp64emu_product_t* p);
 
 int fp64emu_product(const fp64emu_product_t* p, void* workspace, size_t workspace_bytes,

@@ -39,11 +39,25 @@ def _check(dev, kind, batch, M, N, K, P, corr, exact=True):
     ("mm", 1, 250, 500, 131_137, 13, False, True),
     ("mm", 1, 256, 300, 150_000, 15, True, False),
     ("bmm", 2, 24, 16, 135_000, 15, True, True),
-    ("mm", 1, 3, 2, 1_200_000, 15, True, True),
+    ("mm", 1, 40, 24, 600_000, 15, True, True),
+    ("mm", 1, 100, 130, 140_001, 15, True, True),   # 128-row plane tiles: two column tiles
+    ("bmm", 3, 129, 60, 131_200, 14, False, True),
+    ("mm", 1, 3, 2, 1_200_000, 15, True, True),     # past the workspace bound: segmented
     ("mm", 1, 2, 3, 2_096_200, 15, True, True),     # past the whole-K bound: segmented
 ])
 def test_whole_k(dev, kind, batch, M, N, K, P, corr, exact):
     _check(dev, kind, batch, M, N, K, P, corr, exact)
+
+
+def test_whole_k_other_moduli(dev):
+    """A list outside the default one, with an even modulus below 256 (its tie fix), on
+    128-row plane tiles."""
+    A, B = _pair("mm", 1, 70, 90, 132_000, 3, dev)
+    primes = [254, 255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217]
+    got = capi.product("mm", A, B, primes, fill=0x5A)
+    ref, _, _ = capi.run("mm", A, B, primes)
+    torch.cuda.synchronize()
+    assert bits_equal(got.cpu().numpy(), ref.cpu().numpy())
 
 
 # Rows that end inside 64-row groups, 128-row tiles and 256-row tiles.

@@ -39,3 +39,41 @@ def _refusal(batch, M, N, K, P=14, corr=True):
 def test_fused_groups_at_the_dispatch_bound(batch, M, N, K, fused, refused):
     assert _fused(batch, M, N, K) == fused
     assert _refusal(batch, M, N, K) == ("problem too large for one launch" if refused else "")
+
+
+# Past K = 131071: planes of the whole depth, where they are few times the operands or the
+# segmented form's workspace; otherwise the segmented form and no more than it takes.
+@pytest.mark.parametrize("batch,M,N,K,whole", [
+    (1, 300, 200, 200_000, True), (1, 2000, 2000, 150_000, True), (1, 20, 20, 600_000, True),
+    (1, 300, 300, 800_000, True), (1, 129, 300, 131_072, True), (8, 100, 100, 140_000, True),
+    (1, 1, 1, 2_000_000, False), (1, 20, 20, 700_000, False), (1, 30, 30, 1_000_000, False),
+    (1, 20_000, 64, 140_000, False), (1, 2, 3, 2_096_200, False),
+])
+def test_whole_k_workspace_is_bounded(batch, M, N, K, whole):
+    P, corr = fp64_emu.plan_config(K)
+    asked = capi.product_workspace(batch, M, N, K, fp64_emu._PRIMES[:P], corr)
+    segmented = capi.workspace_size(batch, M, N, K, P, corr)
+    assert (asked > segmented) == whole and asked >= segmented
+    assert asked <= max(segmented, min(24 << 30, 5 * max(8 * batch * (M + N) * K, segmented)))
+
+
+def test_whole_k_planes_hold_the_rows_that_are_read():
+    """128 x 128 tiles: planes of 128-row tiles, not 256."""
+    M, N, K, P = 100, 30, 200_000, 15
+    planes = 2 * 128 * (P + 2) * (-(-K // 64) * 64)
+    asked = capi.product_workspace(1, M, N, K, fp64_emu._PRIMES[:P])
+    assert planes < asked < 1.1 * planes
+
+
+def test_whole_k_workspace_fuzz():
+    """Seeded shapes and modulus counts of every depth past 131071, the correction on and off."""
+    rng = np.random.default_rng(5)
+    for _ in range(1500):
+        batch = int(np.exp(rng.uniform(0, np.log(50)))) if rng.random() < 0.3 else 1
+        M, N = (int(np.exp(rng.uniform(0, np.log(5000)))) for _ in range(2))
+        K = int(np.exp(rng.uniform(np.log(131072), np.log(128 * 65536))))
+        P, corr = int(rng.integers(1, 21)), bool(rng.integers(2))
+        asked = capi.product_workspace(batch, M, N, K, fp64_emu._PRIMES[:P], corr)
+        segmented = capi.workspace_size(batch, M, N, K, P, corr)
+        bound = max(segmented, min(24 << 30, 5 * max(8 * batch * (M + N) * K, segmented)))
+        assert asked <= bound, (batch, M, N, K, P, corr)
