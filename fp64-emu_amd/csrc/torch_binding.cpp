@@ -31,18 +31,19 @@ at::Tensor workspace(const at::Tensor& like, size_t bytes) {
   return at::empty({(int64_t)std::max<size_t>(bytes, 1)}, like.options().dtype(at::kByte));
 }
 
-// The full workspace when the caching allocator can provide it; otherwise
-// the largest of full/2, full/4, ... down to the minimum the library accepts
-// (it then runs the rows of A in as few chunks as fit).  Only batch-1 calls
-// with K <= 131071 have a smaller minimum; the others need the full size.
-template <typename Minimum>
-at::Tensor workspace_fit(const at::Tensor& like, size_t full, const Minimum& minimum_size) {
+// The full workspace when the caching allocator can provide it; otherwise the
+// staged form's, where that is smaller (the planes of a whole-K product are
+// several times its segmented ones); otherwise the largest of half, a quarter,
+// ... of that down to the minimum the library accepts (it then runs the rows
+// of A in as few chunks as fit: batch-1 calls with K <= 131071).
+template <typename Size>
+at::Tensor workspace_fit(const at::Tensor& like, size_t full, const Size& size) {
   try {
     return workspace(like, full);
   } catch (const c10::OutOfMemoryError&) {
   }
-  const size_t minimum = minimum_size();
-  for (size_t want = full / 2; want > minimum; want /= 2) {
+  const size_t staged = size(fp64emu_workspace_size), minimum = size(fp64emu_workspace_size_min);
+  for (size_t want = staged < full ? staged : full / 2; want > minimum; want /= 2) {
     try {
       return workspace(like, want);
     } catch (const c10::OutOfMemoryError&) {
@@ -91,8 +92,8 @@ void product(at::Tensor& out, const at::Tensor& A, const at::Tensor& B, int64_t 
   p.exact = exact;
   p.bits = bits;
   p.use_corr = use_corr;
-  at::Tensor ws = workspace_fit(A, fp64emu_product_workspace(&p), [&]() {
-    return fp64emu_workspace_size_min(batch, M, N, K, p.nprimes, use_corr);
+  at::Tensor ws = workspace_fit(A, fp64emu_product_workspace(&p), [&](auto workspace_size) {
+    return workspace_size(batch, M, N, K, p.nprimes, use_corr);
   });
   check_status(fp64emu_product(&p, ws.data_ptr(), (size_t)ws.numel(), current_stream(A)));
 }

@@ -60,6 +60,33 @@ def test_whole_k_other_moduli(dev):
     assert bits_equal(got.cpu().numpy(), ref.cpu().numpy())
 
 
+def test_workspace_fallback_takes_the_staged_size(dev):
+    """A whole-K product that the allocator cannot give its workspace runs segmented in that
+    form's own, not in half of the larger one."""
+    import fp64_emu
+    M, N, K = 300, 300, 400_000
+    A, B = _pair("mm", 1, M, N, K, 5, dev)
+    P, corr = fp64_emu.plan_config(K)
+    full = capi.product_workspace(1, M, N, K, fp64_emu._PRIMES[:P], corr)
+    staged = capi.workspace_size(1, M, N, K, P, corr)
+    assert full > 2.5 * staged
+    want = fp64_emu.mm(A, B)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    held = torch.cuda.memory_reserved()
+    total = torch.cuda.get_device_properties(dev).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((held + 0.7 * full) / total, dev)
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        got = fp64_emu.mm(A, B)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert torch.cuda.max_memory_allocated() - before < staged + (64 << 20)
+    assert bits_equal(got.cpu().numpy(), want.cpu().numpy())
+
+
 # Rows that end inside 64-row groups, 128-row tiles and 256-row tiles.
 @pytest.mark.parametrize("kind,batch,M,N,K,P,corr", [
     ("mm_nt", 1, 1, 1, 1, 14, True),
