@@ -596,24 +596,31 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
                        ? round_up(std::max<int64_t>(N, 1), 128) : L->Np;
 }
 
-// Fused products (fused_kernel): which tile the launch takes.  Against the
-// staged GEMM and reconstruction, a fused group loads its operands from L2 or
-// beyond with little reuse (a 64 x 64 tile reads 32 bytes an output and k-step
-// over 16 slots, a 256 x 256 tile 8), and saves the planes between (36 bytes an
-// output) and a launch.  So it pays for shallow products, and for deeper ones
-// only while they leave the chip idle.  Whole calls, staged / 32 x 32 / 64 x 32
-// / 64 x 64, us (mm or bmm, 14 + correction):
-//   64^3            21.1  17.6  18.8  22.8    1024^2 x 256    41.0  34.4  34.5  32.5
-//   128^2 x 512     24.7  22.2  25.7  31.0    1024^3          59.8  65.9  59.3  49.6
-//   128^2 x 1024    25.0  27.9  35.3  43.0    1024^2 x 2048   87.3   115  97.0  79.3
-//   256^2 x 1024    35.8  31.7  37.6  44.0    2000^2 x 512     101   110  97.7  95.9
-//   256^2 x 2048    38.3  43.1  52.6  64.2    2000^2 x 1000    132   200   174   143
-//   512^3           31.8  27.2  30.7  35.4    3000^2 x 256     145   129   120   145
-//   512^2 x 4096    78.4  73.7  97.8   119    64 x 256^3       136   114   108   118
-//   768^3           50.9  48.4  47.6  44.8    8 x 512^2 x 1024 121   138   123   108
-//   768^2 x 1536    64.6  74.3  72.6  64.1    16 x 512^3       138   141   128   123
-//   1500^2 x 256    58.0  50.1  51.0  58.8    32 x 512^3       267   315   290   301
-//   1500^2 x 700    83.4  97.8  88.0  90.3    64 x 512^2 x 128 263   240   201   249
+// Fused products (fused_kernel): which tile the launch takes, if any.  Against
+// the staged GEMM and reconstruction, a fused group loads its operands from L2
+// or beyond with little reuse (a 64 x 64 tile reads 32 bytes an output and
+// k-step over 16 slots, a 256 x 256 tile 8), and saves the planes between (36
+// bytes an output) and a launch.  So it pays for shallow products, and for
+// deeper ones only while the staged form leaves the chip idle or works on
+// padding: fused_tile_choice takes the tile from the sizes, fused_pays keeps
+// it where the estimate of its launch is below that of the staged ones.  Whole
+// calls, staged / 32 x 32 / 64 x 32 / 64 x 64, us (bmm, * the rule's; 14
+// moduli and the correction, below the line 13 without):
+//   64^2 x 128      18.6  13.9* 15.3  18.9    1024^3          62.9  66.0  58.2  50.1*
+//   128^2 x 512     21.9  19.7* 23.1  28.3    1024^2 x 2048   85.6   114  97.3  79.0*
+//   128^2 x 1024    22.4* 25.1  31.4  39.3    1408^2 x 512    66.9  66.7  60.8  61.2*
+//   256^2 x 1024    33.4* 29.3  34.8  41.3    1408^2 x 1024   86.3   113  96.6  88.5*
+//   256^2 x 2048    37.6* 42.3  51.2  62.6    1536^2 x 256    56.6  50.4  47.3* 57.3
+//   512^3           29.6  25.3* 28.1  32.9    2048^2 x 1024    132*  202   163   142
+//   512^2 x 4096    78.2* 75.6  99.6   119    16 x 256^2 x 1024 98.7 96.6  87.1  82.3*
+//   576^2 x 1024    40.1* 43.8  39.6  46.7    32 x 256^2 x 1024 195   237   213   204*
+//   640^2 x 1536    49.6* 57.8  51.8  60.4    8 x 200^2 x 2048 92.6*  112   101   109
+//   768^3           49.8  46.2  46.1  42.3*   25 x 120^2 x 1536 111*  131   133   140
+//   960^2 x 2048    85.0*  120   115  96.3    64 x 64^2 x 2560  309   218*  239   266
+//   ----
+//   512^3           25.6  22.9* 26.2  31.0    1000^2 x 2048   81.5  97.9  85.6  72.1*
+//   640^2 x 1024    33.1* 39.7  37.9  44.1    1792^2 x 512    70.3* 82.8  76.8  87.8
+//   768^2 x 1024    36.8* 48.3  48.5  45.6    256 x 64^2 x 2048 749   549   547   547*
 enum FusedTile { kFusedNone, kFused32x32, kFused64x32, kFused64x64 };
 constexpr int kFusedThreads = 512;
 
@@ -642,12 +649,73 @@ FusedTile fused_tile_choice(const fp64emu_layout_t& L) {
   return kFusedNone;
 }
 
-// The fused launch of a product, or none where its groups pass the 2^32 - 1
-// work-items of a dispatch: the staged form's launches (of fewer work-items an
-// output where rows end early in their tiles) may still hold such a product.
+// Panel rows an XCD's L2 fetches per tile where it takes 32 tiles in a row (8
+// tile rows by 4 columns, or whole members) of TM x TN tiles of r x c.
+double panel_rows(int64_t TM, int64_t TN, int64_t r, int64_t c) {
+  double m = (double)TM, n = (double)TN;
+  if (TM * TN >= 32) {
+    m = std::min(m, 8.0);
+    n = std::min(n, 32.0 / m);
+  }
+  return r / n + c / m;
+}
+
+// Estimates of the fused launch and of the staged GEMM and reconstruction, in
+// us, fitted to calls timed both ways (13 and 14 moduli, with and without the
+// correction, 1 to 64 k-steps, 1 to 300 members, up to 4 rounds of 64 x 64
+// tiles).  Staged: rounds of groups, whole and fractional, each of its k-steps,
+// and a cost per group's end.  Fused: rounds of groups (of the small tiles two
+// share a CU, whose k-steps then take 1.08 us for both instead of 0.56), each of
+// its k-steps (without the correction's wave a wave of the large tile holds two
+// residue slots one after the other).  Either way not less than the operands
+// that the XCDs' L2s fetch take at 10 TB/s: of a full chunk of 256 groups an XCD
+// takes 32 tiles in a row; the fused groups past the last full chunk go round
+// the XCDs and share little (of one matrix of at least 8 tile rows, an XCD keeps
+// to one in 8).  kOthers: the reconstruction's launch and the planes between
+// (more of them with a K-split).
+// Of 2208 timed calls the rule without these estimates took 258 more than 2%
+// slower than staged (5 x 221 x 216 x 3776 in twice the time), with them 40 (at
+// most 12%).
+bool fused_pays(const fp64emu_layout_t& L, FusedTile t) {
+  if (L.gemm_run > 1) return true;   // slot runs: many tiles, shallow enough
+  const double kOthers = L.ksplit > 1 ? 4.5 : 3.6;
+  constexpr double kFetchBytesPerUs = 10.0e6;
+  constexpr struct { double step, round_step, group; } kStaged[3] = {
+      {0.31, 0.25, 4.6}, {0.27, 0.56, 7.8}, {0.05, 0.56, 13.7}};   // 128 x 128, 256 x 128, 256 x 256
+  const int64_t nkt = L.Kp / kTileK, moduli = L.nprimes + (L.use_corr ? 2 : 0);
+  const double panel_us = (double)(kTileK * nkt * moduli) / kFetchBytesPerUs;   // of one row of a panel
+
+  const int64_t rows = L.gemm_tile_rows, cols = L.gemm_tile_cols;
+  const int form = rows == 128 ? 0 : cols == 128 ? 1 : 2;
+  const int64_t sTM = rows == 128 ? (L.M + 127) / 128 : L.Mp / kTileR;
+  const int64_t sTN = cols == 128 ? (L.N + 127) / 128 : L.Np / kTileR;
+  const int64_t tiles = L.batch * sTM * sTN, groups = tiles * L.ksplit * moduli;
+  const int64_t slots = cols == 128 ? 2 * kCUs : kCUs, steps = (nkt + L.ksplit - 1) / L.ksplit;
+  const double fill = (double)groups / slots, rounds = (double)((groups + slots - 1) / slots);
+  const double staged = std::max(fill * (kStaged[form].step * steps + kStaged[form].group) +
+                                     rounds * kStaged[form].round_step * steps,
+                                 tiles * panel_rows(sTM, sTN, rows, cols) * panel_us);
+
+  const int64_t r = fused_rows(t), c = fused_cols(t), TM = (L.M + r - 1) / r, TN = (L.N + c - 1) / c;
+  const int64_t all = L.batch * TM * TN, n = (all + kCUs - 1) / kCUs, past = all % kCUs;
+  double fused;
+  if (t == kFused64x64) fused = n * ((L.use_corr ? 1.04 : 1.22) * nkt + 5.0);
+  else if (t == kFused64x32) fused = (n / 2 * 1.59 + n % 2 * 0.87) * nkt + 1.8 * n;
+  else fused = (n / 2 * 1.08 + n % 2 * 0.56) * nkt + 0.9 * n;
+  const double fetched = (all - past) * panel_rows(TM, TN, r, c) +
+                         past * (L.batch == 1 && TM >= 8 ? c + r / 4.0 : (double)(r + c));
+  return std::max(fused, fetched * panel_us) < staged + kOthers;
+}
+
+// The fused launch of a product, or none where it would not pay or its groups
+// pass the 2^32 - 1 work-items of a dispatch: the staged form's launches (of
+// fewer work-items an output where rows end early in their tiles) may still
+// hold such a product.
 FusedTile fused_tile(const fp64emu_layout_t& L) {
   const FusedTile t = fused_tile_choice(L);
-  return t != kFusedNone && fused_groups(L, t) > (int64_t)0xFFFFFFFFu / kFusedThreads ? kFusedNone : t;
+  if (t == kFusedNone || fused_groups(L, t) > (int64_t)0xFFFFFFFFu / kFusedThreads || !fused_pays(L, t))
+    return kFusedNone;
+  return t;
 }
 
 // The layout of fp64emu_product, which leaves no stage for inspection: rows

@@ -77,3 +77,19 @@ def test_whole_k_workspace_fuzz():
         segmented = capi.workspace_size(batch, M, N, K, P, corr)
         bound = max(segmented, min(24 << 30, 5 * max(8 * batch * (M + N) * K, segmented)))
         assert asked <= bound, (batch, M, N, K, P, corr)
+
+
+# Where fused products lost to the staged form, and where they gain (14 and 13 moduli:
+# with the correction and without; the columns are whether the call runs fused).
+@pytest.mark.parametrize("batch,M,N,K,with_corr,without", [
+    (1, 64, 64, 64, True, True), (1, 333, 501, 777, True, True), (1, 512, 512, 512, True, True),
+    (1, 1024, 1024, 1024, True, True), (64, 256, 256, 256, True, True), (1, 4000, 4000, 256, True, True),
+    (64, 64, 64, 2560, True, True), (1, 1000, 1000, 2048, True, True),
+    (1, 640, 640, 1536, False, False), (1, 480, 500, 3500, False, False), (8, 200, 200, 2048, False, False),
+    (24, 128, 128, 2048, False, False), (5, 221, 216, 3776, False, False), (1, 960, 960, 2048, False, False),
+    (6, 448, 320, 1984, False, False), (25, 120, 120, 1536, False, False),
+    (1, 768, 768, 768, True, False), (1, 2000, 2000, 512, True, False),
+])
+def test_fused_only_where_it_pays(batch, M, N, K, with_corr, without):
+    assert _fused(batch, M, N, K, 14, True) == with_corr
+    assert _fused(batch, M, N, K, 13, False) == without
