@@ -609,7 +609,7 @@ void make_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool cor
 //   64^2 x 128      18.6  13.9* 15.3  18.9    1024^3          62.9  66.0  58.2  50.1*
 //   128^2 x 512     21.9  19.7* 23.1  28.3    1024^2 x 2048   85.6   114  97.3  79.0*
 //   128^2 x 1024    22.4* 25.1  31.4  39.3    1408^2 x 512    66.9  66.7  60.8  61.2*
-//   256^2 x 1024    33.4* 29.3  34.8  41.3    1408^2 x 1024   86.3   113  96.6  88.5*
+//   256^2 x 1024    33.4  29.3* 34.8  41.3    1408^2 x 1024   86.3   113  96.6  88.5*
 //   256^2 x 2048    37.6* 42.3  51.2  62.6    1536^2 x 256    56.6  50.4  47.3* 57.3
 //   512^3           29.6  25.3* 28.1  32.9    2048^2 x 1024    132*  202   163   142
 //   512^2 x 4096    78.2* 75.6  99.6   119    16 x 256^2 x 1024 98.7 96.6  87.1  82.3*
@@ -736,32 +736,46 @@ bool whole_k_fits(const fp64emu_layout_t& whole, const fp64emu_layout_t& segment
 // Whole rounds: products of fewer 256 x 256 tiles than CUs whose tiles x slots
 // (the correction as two slots, each as deep as a residue's) come to whole
 // rounds of the chip run one slot per group without a K-split, every CU the
-// same k-steps.  The staged forms give such products 256 x 128 tiles, K-splits
-// or a double-length correction slot, for shapes whose tiles do not come out
-// even; here those cost operand traffic, split planes or a ragged last round.
-// Staged / whole rounds, whole calls, us (14 + correction: 16 slots a tile):
-//   1024^2 x 2560  (1 round)  107 /  95    2048^2 x 3000    (4)   300 /  281
-//   1024^2 x 16000 (1)        452 / 419    2048^2 x 8192    (4)   700 /  636
-//   1280 x 1536 x 3000 (1.9)  190 / 180    16 x 512^2 x 8192 (4) 1397 / 1323
-//   1024 x 2048 x 3000 (2)    187 / 163    16 x 256^2 x 32768 (1) 2632 / 2398
-//   1536 x 2048 x 8192 (3)    566 / 504    3000^2 x 8192    (9)  1249 / 1210
-// Shallow products need more rounds to gain: 1024^2 x 1536 (1) 65 / 77,
-// 1280 x 1536 x 2000 (1.9) 127 / 141, 2000^2 x 1000 (4) 132 / 135, 1024 x
-// 2048 x 2048 (2) 130 / 127, 2048^2 x 1500 (4) 172 / 168, 2000^3 (4) 217 / 208;
-// at 256 tiles and more the fused correction is balanced already (4096^2 x
-// 8192 1963 / 1992), and off whole rounds the staged forms stay (1024 x 1280 x
-// 3000, 1.25 rounds, 132 / 140).
+// same k-steps.  The staged forms give such products 256 x 128 tiles,
+// K-splits or a double-length correction slot, for shapes whose tiles do not
+// come out even; here those cost operand traffic, split planes or a ragged last
+// round.  Staged / whole rounds, whole calls, us (14 + correction: 16 slots a
+// tile; the rounds in brackets):
+//   1024^2 x 2560  (1)         106 / 94     2048^2 x 3000   (4)     299 / 277
+//   1024^2 x 16384 (1)         459 / 430    2048^2 x 8192   (4)     706 / 633
+//   1280 x 1536 x 4096 (1.9)   241 / 223    16 x 512^2 x 8192 (4)  1390 / 1309
+//   1024 x 2048 x 3000 (2)     184 / 163    2816^2 x 4096   (7.6)   623 / 592
+//   1536 x 2048 x 8192 (3)     577 / 499    3072^2 x 8192   (9)    1293 / 1236
+// From about 150 tiles on (kFusedCorrTiles) the fused correction evens out among
+// many rounds, and as two slots only reads its planes apart: even at 12 and 15
+// rounds (3072 x 4096 x 2560 615 / 614, 4096 x 3840 x 4096 1069 / 1081), slower
+// between them (3328^2 x 2560 529 / 553, 3500^2 x 2560 609 / 645); whole rounds
+// stay there to 32 k-steps, where the staged tiles are narrow (4096 x 3840 x
+// 2048 648 / 641; without the correction 3500^2 x 1600 370 / 349).  Under 40 k-steps
+// products of one matrix gain from 32 on in three rounds and more (2048^2 x
+// 2048 211 / 211, x 2304 241 / 226; 1000 x 4000 x 1536 175 / 184) and from 36
+// in two (1024 x 2048 x 2048 128 / 131, x 2304 154 / 136), members, whose
+// staged tiles share less, earlier (8 x 512^2 x 2048 (2) 234 / 209, 16 x 512^2
+// x 1536 (4) 313 / 304).  Rounds not quite whole lose to the K-split where it is
+// long and the rounds few: 1280 x 1536 (1.9) x 8192 399 / 409, x 32768 1383 /
+// 1499; and off them the staged forms stay (1024 x 1280 x 3000, 1.25 rounds,
+// 132 / 140).
+constexpr int64_t kFusedCorrTiles = 150;
+
 bool whole_rounds(const fp64emu_layout_t& L) {
   if (L.deep || L.nchunk != 1) return false;
   if (L.Np / kTileR >= 2 && L.N % kTileR != 0 && L.N % kTileR <= 128) return false;   // a mixed launch
   const int64_t rows128 = round_up(std::max<int64_t>(L.M, 1), 128), cols128 = round_up(std::max<int64_t>(L.N, 1), 128);
   if (rows128 * cols128 * 11 < L.Mp * L.Np * 10) return false;   // mostly padding at 256
   const int64_t tiles = L.batch * (L.Mp / kTileR) * (L.Np / kTileR);
-  if (tiles >= kCUs) return false;
+  if (tiles >= kCUs) return false;   // (the fused correction is balanced: 4096^2 x 8192 1963 / 1992)
   const int64_t units = tiles * (L.nprimes + (L.use_corr ? 2 : 0));
   const int64_t n = (units + kCUs - 1) / kCUs, nkt = L.Kp / kTileK;
+  const bool whole = units * 100 >= n * kCUs * 99;
+  if (L.use_corr && tiles > kFusedCorrTiles && !(whole && nkt <= kRunMaxSteps)) return false;
+  if (nkt >= 128 && n < 4) return whole;
   if (nkt >= 40) return units * 100 >= n * kCUs * 93;
-  return units * 100 >= n * kCUs * 99 && nkt >= (n >= 3 ? 24 : 32) && n >= 2;
+  return whole && n >= 2 && nkt >= (L.batch > 1 ? (n >= 3 ? 24 : 32) : (n >= 3 ? 32 : 36));
 }
 
 void make_product_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool corr,

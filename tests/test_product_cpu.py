@@ -93,3 +93,18 @@ def test_whole_k_workspace_fuzz():
 def test_fused_only_where_it_pays(batch, M, N, K, with_corr, without):
     assert _fused(batch, M, N, K, 14, True) == with_corr
     assert _fused(batch, M, N, K, 13, False) == without
+
+
+# Whole rounds (the correction as two slots) where they gain, the staged form elsewhere:
+# many tiles, a long K-split against rounds not quite whole, few k-steps.
+@pytest.mark.parametrize("batch,M,N,K,rounds", [
+    (1, 1024, 1024, 2560, True), (1, 2048, 2048, 3000, True), (1, 2000, 2000, 2000, True),
+    (16, 512, 512, 8192, True), (16, 512, 512, 1536, True), (8, 512, 512, 2048, True),
+    (1, 3072, 3072, 4096, True), (1, 1280, 1536, 4096, True), (1, 4096, 3840, 2000, True),
+    (1, 3500, 3500, 2560, False), (1, 3840, 3840, 2600, False), (1, 4096, 3840, 4096, False),
+    (1, 1280, 1536, 8192, False), (1, 1280, 1536, 32768, False),
+    (1, 1000, 4000, 1536, False), (1, 1024, 2048, 2048, False),
+])
+def test_whole_rounds_only_where_they_pay(batch, M, N, K, rounds):
+    asked = capi.product_workspace(batch, M, N, K, fp64_emu._PRIMES[:14])
+    assert (asked != capi.workspace_size(batch, M, N, K, 14, True)) == rounds
