@@ -142,9 +142,10 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-def product(kind, A, B, primes, exact=True, bits=53, use_corr=True, fill=None):
+def product(kind, A, B, primes, exact=True, bits=53, use_corr=True, fill=None, ws_bytes=None):
     """fp64emu_product on checked device tensors: the call of the torch ops.
-    `fill`: a byte to fill the workspace with first."""
+    `fill`: a byte to fill the workspace with first; `ws_bytes`: its size, the
+    one the call asks for by default."""
     primes = np.ascontiguousarray(np.asarray(primes, dtype=np.int32))
     batched, nt = kind in ("bmm", "bmm_nt"), kind.endswith("_nt")
     if A.dim() != (3 if batched else 2) or B.dim() != A.dim() or (batched and B.shape[0] != A.shape[0]):
@@ -160,7 +161,7 @@ def product(kind, A, B, primes, exact=True, bits=53, use_corr=True, fill=None):
     out = torch.empty((batch, M, N) if batched else (M, N), dtype=torch.float64, device=A.device)
     p = Product(out.data_ptr(), A.data_ptr(), B.data_ptr(), batch, M, N, K, int(nt),
                 primes.ctypes.data, primes.size, int(bool(exact)), int(bits), int(bool(use_corr)))
-    n = lib().fp64emu_product_workspace(ctypes.byref(p))
+    n = lib().fp64emu_product_workspace(ctypes.byref(p)) if ws_bytes is None else ws_bytes
     ws = torch.empty(max(int(n), 1), dtype=torch.uint8, device=A.device)
     if fill is not None:
         ws.fill_(fill)

@@ -99,17 +99,53 @@ def test_unpadded_rows(dev, kind, batch, M, N, K, P, corr):
     _check(dev, kind, batch, M, N, K, P, corr)
 
 
-# Whole rounds: item streams (33 to 64 k-steps) and single items (more), the rounds not
-# quite whole, no correction (13 slots), members, ragged edges, both combines.
+# Whole rounds: single items (fewer than 512 units, or more than 64 k-steps) and item
+# streams (512 units and more of at most 64 k-steps) with the correction as two slots, the
+# rounds not quite whole, no correction (13 slots), members, ragged edges, both combines.
 @pytest.mark.parametrize("kind,batch,M,N,K,P,corr,exact", [
     ("mm_nt", 1, 1000, 1024, 2600, 14, True, True),      # 1 round
     ("mm", 1, 1279, 1500, 2561, 14, True, True),         # 1.9 rounds
     ("bmm_nt", 19, 250, 256, 2700, 13, False, True),     # 247 of 256 units
     ("bmm", 16, 256, 230, 4200, 14, True, False),        # past the streams' depth
     ("mm", 1, 1792, 2000, 1537, 14, True, True),         # 3.5 rounds: staged
+    ("mm_nt", 1, 2000, 2000, 2000, 14, True, True),      # streams: 4 rounds of 32 k-steps
+    ("mm", 1, 2048, 2030, 3000, 14, True, False),        # of 47
+    ("mm_nt", 1, 1000, 4000, 4096, 14, True, True),      # of 64, the most
+    ("mm", 1, 1500, 2048, 2300, 14, True, True),         # 3 rounds of 36
+    ("bmm_nt", 16, 500, 512, 1536, 14, True, True),      # members, 24 k-steps
+    ("bmm", 8, 512, 500, 2100, 14, True, True),          # 2 rounds of 33
 ])
 def test_whole_rounds(dev, kind, batch, M, N, K, P, corr, exact):
+    primes = O.PRIMES[:P]
+    if corr and batch * (-(-M // 256)) * (-(-N // 256)) * (P + 2) % 256 == 0:   # whole: one corr plane more, or no split
+        assert capi.product_workspace(batch, M, N, K, primes) != capi.workspace_size(batch, M, N, K, P, True)
     _check(dev, kind, batch, M, N, K, P, corr, exact)
+
+
+# On a workspace shorter than it asks for the call runs as the staged entry points do, in
+# row chunks where it must: a byte short, the staged size, the minimum, and refused below.
+@pytest.mark.parametrize("kind,batch,M,N,K,P", [
+    ("mm", 1, 1000, 1024, 1000, 14),         # fused: less than any staged form asks for
+    ("mm_nt", 1, 2000, 2048, 3000, 14),      # whole rounds: staged, then chunked
+    ("bmm", 16, 512, 512, 1536, 14),         # members: staged, never chunked
+    ("mm", 1, 40, 24, 140_000, 15),          # whole K: segmented
+    ("mm", 1, 300, 600, 131_072, 15),
+])
+def test_shorter_workspace(dev, kind, batch, M, N, K, P):
+    print(f"case shorter workspace {kind} b={batch} {M}x{N}x{K}", flush=True)
+    A, B = _pair(kind, batch, M, N, K, 7, dev)
+    primes = O.PRIMES[:P]
+    asked = capi.product_workspace(batch, M, N, K, primes, nt=kind.endswith("_nt"))
+    staged = capi.workspace_size(batch, M, N, K, P, True)
+    least = capi.workspace_size_min(batch, M, N, K, P, True)
+    ref, _, _ = capi.run(kind, A, B, primes)
+    for size in sorted({asked, asked - 256, asked + 4096, staged, staged - 256, (staged + least) // 2, least}):
+        if size >= min(asked, least):
+            got = capi.product(kind, A, B, primes, fill=0x5A, ws_bytes=size)
+            torch.cuda.synchronize()
+            assert bits_equal(got.cpu().numpy(), ref.cpu().numpy()), size
+    with pytest.raises(capi.CapiError, match="workspace too small"):
+        capi.product(kind, A, B, primes, ws_bytes=min(asked, least) - 256)
 
 
 # Fused GEMM and reconstruction: each tile (32 x 32, 64 x 32, 64 x 64), edges inside and
@@ -119,7 +155,8 @@ def test_whole_rounds(dev, kind, batch, M, N, K, P, corr, exact):
     ("mm", 1, 1, 1, 1), ("mm_nt", 1, 16, 17, 64), ("mm", 1, 33, 31, 65), ("bmm_nt", 3, 47, 50, 200),
     ("mm_nt", 1, 512, 512, 64 * 17),                                           # 32 x 32, 256 tiles
     ("bmm", 5, 400, 410, 3 * 64 + 5), ("bmm_nt", 40, 129, 200, 257),           # 64 x 32
-    ("mm", 1, 800, 900, 700), ("bmm_nt", 12, 500, 300, 500), ("mm_nt", 1, 1025, 1000, 1100),   # 64 x 64
+    ("mm", 1, 800, 900, 700), ("bmm_nt", 12, 500, 300, 500), ("mm_nt", 1, 1025, 1000, 1100),   # 64 x 64 (the last: staged)
+    ("mm", 1, 1000, 1024, 2000), ("mm_nt", 1, 1400, 1390, 600),   # 64 x 64 of 32 k-steps; past one round
 ])
 @pytest.mark.parametrize("P,corr,exact", [(14, True, True), (13, False, True), (14, True, False), (13, True, False),
                                           (14, False, True)])
