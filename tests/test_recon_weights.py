@@ -1,17 +1,24 @@
-"""CPU tier: the remainder-weight combine of the reconstruction (crt4 and
-crt_combine in fp64emu.hip), restated operation by operation in correctly
-rounded float64 and compared with exact integers: three 39-bit slices of the
-weights, any residue representatives (a K-split's sums among them), the
+"""CPU tier: the remainder-weight combine of the reconstruction (crt_values and
+crt_combine in remainder_weights.h) against exact integers: three 39-bit slices
+of the weights, any residue representatives (a K-split's sums among them), the
 correction, and a single rounding -- at range ends, ties and cancellations.
-Tolerance: none (the same bits)."""
+The kernels' own code, compiled for the host, and its operations restated in
+correctly rounded float64 (with the slices' bounds).  Tolerance: none (the same
+bits)."""
+import ctypes
 import math
+import os
 import random
+import subprocess
 from fractions import Fraction
 
 import pytest
 
 import oracle as O
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "fp64-emu_amd", "csrc")
+HIPCC = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
 BITS = 39
 
 
@@ -60,15 +67,13 @@ def _combine(s, cv, cshift, M):
     return h2 + y
 
 
-@pytest.mark.parametrize("P,fold", [(12, 1), (13, 1), (14, 1), (15, 1), (13, 16), (14, 16), (15, 8)])
-def test_weight_combine_rounds_once(P, fold):
+FOLDS = [(12, 1), (13, 1), (14, 1), (15, 1), (13, 16), (14, 16), (15, 8)]
+
+
+def _cases(P, fold):
+    """(X, cv, cshift, residues): X = sum of the residues at their weights, mod M."""
     primes = [int(p) for p in O.PRIMES[:P]]
-    M, W = _weights(primes)
-    slices = [_slices(w) for w in W]
-    for i in range(3):   # every partial sum, before and after q M, is an exact float64
-        bound = fold * sum(p // 2 * abs(s[i]) for p, s in zip(primes, slices))
-        q = fold * sum(p // 2 * abs(w) for p, w in zip(primes, W)) // M + 1
-        assert bound + q * abs(_slices(M)[i]) < 2 ** 53
+    M, _ = _weights(primes)
     rng = random.Random(100 * P + fold)
     lim = 36 * M // 100
     for it in range(600):
@@ -89,6 +94,72 @@ def test_weight_combine_rounds_once(P, fold):
                      for _ in range(fold - 1)]
             last = (X - sum(parts)) % p
             r.append(sum(parts) + (last - p if last > (p - 1) // 2 else last))
+        yield X, cv, cs, r
+
+
+def _same(a, b):
+    return a == b and math.copysign(1.0, a) == math.copysign(1.0, b)
+
+
+@pytest.mark.parametrize("P,fold", FOLDS)
+def test_weight_combine_rounds_once(P, fold):
+    primes = [int(p) for p in O.PRIMES[:P]]
+    M, W = _weights(primes)
+    slices = [_slices(w) for w in W]
+    for i in range(3):   # every partial sum, before and after q M, is an exact float64
+        bound = fold * sum(p // 2 * abs(s[i]) for p, s in zip(primes, slices))
+        q = fold * sum(p // 2 * abs(w) for p, w in zip(primes, W)) // M + 1
+        assert bound + q * abs(_slices(M)[i]) < 2 ** 53
+    for X, cv, cs, r in _cases(P, fold):
         s = [float(sum(Fraction(ri) * Fraction(si[i]) for ri, si in zip(r, slices))) for i in range(3)]
-        got, want = _combine(s, cv, cs, M), float(Fraction(X + (cv << cs)))
-        assert got == want and math.copysign(1.0, got) == math.copysign(1.0, want), (X, cv, cs)
+        assert _same(_combine(s, cv, cs, M), float(Fraction(X + (cv << cs)))), (X, cv, cs)
+
+
+HOST = """
+#include "remainder_weights.h"
+template <int kP> static double value(const int* r, double cv, int cshift, int sh) {
+  const double cvs[1] = {cv};
+  const int shs[1] = {sh};
+  double out[1];
+  crt_values<kP, 1>([&](int t, int) { return r[t]; }, cvs, cshift, shs, out);
+  return out[0];
+}
+extern "C" double host_value(int P, const int* r, double cv, int cshift, int sh) {
+  switch (P) {
+    case 12: return value<12>(r, cv, cshift, sh);
+    case 13: return value<13>(r, cv, cshift, sh);
+    case 14: return value<14>(r, cv, cshift, sh);
+    default: return value<15>(r, cv, cshift, sh);
+  }
+}
+extern "C" int host_exact(int P, int fold) { return crt_exact(P, fold); }
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    d = tmp_path_factory.mktemp("weights")
+    (d / "host.hip").write_text(HOST)
+    subprocess.run([HIPCC, "--offload-host-only", "-O1", "-std=c++17", "-fPIC", "-ffp-contract=off", "-shared",
+                    f"-I{CSRC}", f"-I{ROOT}/include", str(d / "host.hip"), "-o", str(d / "host.so")], check=True)
+    L = ctypes.CDLL(str(d / "host.so"))
+    L.host_value.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_double, ctypes.c_int, ctypes.c_int]
+    L.host_value.restype = ctypes.c_double
+    return L
+
+
+@pytest.mark.parametrize("P,fold", FOLDS)
+def test_compiled_combine_rounds_once(host, P, fold):
+    assert host.host_exact(P, fold)
+    for i, (X, cv, cs, r) in enumerate(_cases(P, fold)):
+        sh = (0, -7, -60, 40)[i % 4]
+        got = host.host_value(P, (ctypes.c_int * P)(*r), float(cv), cs, sh)
+        assert _same(got, math.ldexp(float(Fraction(X + (cv << cs))), sh)), (X, cv, cs, sh)
+
+
+def test_compiled_combine_bounds(host):
+    """Exact for sums of residues to sixteen splits at 12 to 14 moduli, to eight at 15; no
+    other modulus count."""
+    exact = {(P, f) for P in range(1, 21) for f in (1, 2, 4, 8, 16) if host.host_exact(P, f)}
+    want = {(P, f) for P in (12, 13, 14) for f in (1, 2, 4, 8, 16)} | {(15, f) for f in (1, 2, 4, 8)}
+    assert exact == want
