@@ -2952,27 +2952,24 @@ __device__ __forceinline__ double i128_to_f64(int64_t hi, uint64_t lo, int sh64)
 
 // One element's value from its Horner group values a0, a1, a2 (ng of them
 // used), the group products m0, m1 and the correction sum cv, scaled by 2^sh.
-// short_top: a1 + m1 a2 fits 63 bits.
 template <bool kExact>
 __device__ __forceinline__ double combine_groups(const long long a0, const long long a1, const long long a2,
-                                                 const int ng, const bool short_top, const long long m0,
-                                                 const long long m1, const int64_t cv, const int cshift,
-                                                 const int sh) {
+                                                 const int ng, const long long m0, const long long m1,
+                                                 const int64_t cv, const int cshift, const int sh) {
   if constexpr (kExact) {
-    // X = a0 + M0 (a1 + M1 a2) as a 128-bit word pair (hi, lo).  The one
-    // or two group products of the usual plans (at most 15 moduli: group 2
-    // holds at most one digit, so a1 + M1 a2 fits 63 bits) take
-    // mul_add_wide's four 32 x 32 -> 64 multiply-adds; longer lists take
-    // the general 128-bit product (the true X stays below 2^127, so the
-    // products wrap modulo 2^128 harmlessly).
+    // X = a0 + M0 (a1 + M1 a2) as a 128-bit word pair (hi, lo): the exact
+    // combine of 16 to 20 default moduli (three groups), of fewer than 12, of
+    // other lists and of K-segmented sums (12 to 15 default moduli otherwise
+    // take crt_values).  Two groups take mul_add_wide's four 32 x 32 -> 64
+    // multiply-adds; three the general 128-bit product (the true X stays below
+    // 2^127, so the products wrap modulo 2^128 harmlessly).
     uint64_t lo;
     int64_t hi;
     if (ng == 1) {
       lo = (uint64_t)a0;
       hi = a0 >> 63;
-    } else if (ng == 2 || short_top) {
-      const int64_t top = ng == 2 ? a1 : (int64_t)((uint64_t)a2 * (uint64_t)m1) + a1;
-      mul_add_wide(top, (uint64_t)m0, a0, lo, hi);
+    } else if (ng == 2) {
+      mul_add_wide(a1, (uint64_t)m0, a0, lo, hi);
     } else {
       i128 acc = (i128)a2 * (i128)(uint64_t)m1 + a1;
       acc = acc * (i128)(uint64_t)m0 + a0;
@@ -2995,8 +2992,9 @@ __device__ __forceinline__ double combine_groups(const long long a0, const long 
 }
 
 // Four elements (the bytes of the residue words w[0 .. kP)) of a product over
-// the default modulus list: Garner digits, Horner and the exact or float64
-// combine with the correction sums cv, scaled by 2^sh[e].
+// the default modulus list: Garner digits, Horner and the float64 combine with
+// the correction sums cv (at 16 moduli and more the exact one too), scaled by
+// 2^sh[e].
 template <bool kExact, int kP>
 __device__ __forceinline__ void reconstruct4(const uint32_t (&w)[kMaxP], const int64_t (&cv)[4],
                                              const int cshift, const int (&sh)[4], double (&val)[4]) {
@@ -3088,8 +3086,8 @@ __device__ __forceinline__ void reconstruct4(const uint32_t (&w)[kMaxP], const i
   constexpr int ng = (kP + 6) / 7;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    val[e] = combine_groups<kExact>(ag[e][0], ag[e][1], ag[e][2], ng, kP == 15 || ng < 3, kDefaultM64[0],
-                                    kDefaultM64[1], cv[e], cshift, sh[e]);
+    val[e] = combine_groups<kExact>(ag[e][0], ag[e][1], ag[e][2], ng, kDefaultM64[0], kDefaultM64[1],
+                                    cv[e], cshift, sh[e]);
 }
 
 struct ReconCore {
@@ -3421,7 +3419,7 @@ reconstruct_kernel(ReconArgs<kP == 0> a) {
     // Every group ends on its position-0 digit, an int64 step, so ag holds
     // the group value whatever the group's digit count.
     store_at<double>(oblk + e * a.N, olane,
-                     combine_groups<kExact>(ag[e][0], ag[e][1], ag[e][2], ng, false, tab_m64(0), tab_m64(1),
+                     combine_groups<kExact>(ag[e][0], ag[e][1], ag[e][2], ng, tab_m64(0), tab_m64(1),
                                             (int64_t)cv[e], cshift, -(sai[e] + sj)));
   }
 }
