@@ -735,9 +735,10 @@ bool whole_k_fits(const fp64emu_layout_t& whole, const fp64emu_layout_t& segment
 // 2048 648 / 641; without the correction 3500^2 x 1600 370 / 349).  Under 40 k-steps
 // products of one matrix gain from 32 on in three rounds and more (2048^2 x
 // 2048 211 / 211, x 2304 241 / 226; 1000 x 4000 x 1536 175 / 184) and from 36
-// in two (1024 x 2048 x 2048 128 / 131, x 2304 154 / 136), members, whose
-// staged tiles share less, earlier (8 x 512^2 x 2048 (2) 234 / 209, 16 x 512^2
-// x 1536 (4) 313 / 304).  Rounds not quite whole lose to the K-split where it is
+// in two (1024 x 2048 x 2048 128 / 131, x 2304 154 / 136); earlier members,
+// whose staged tiles share less (8 x 512^2 x 2048 (2) 234 / 209, 16 x 512^2 x
+// 1536 (4) 313 / 304), and products without the correction, which splits into
+// nothing more there (3584^2 x 1536 349 / 340).  Rounds not quite whole lose to the K-split where it is
 // long and the rounds few: 1280 x 1536 (1.9) x 8192 399 / 409, x 32768 1383 /
 // 1499; and off them the staged forms stay (1024 x 1280 x 3000, 1.25 rounds,
 // 132 / 140).
@@ -756,7 +757,8 @@ bool whole_rounds(const fp64emu_layout_t& L) {
   if (L.use_corr && tiles > kFusedCorrTiles && !(whole && nkt <= kRunMaxSteps)) return false;
   if (nkt >= 128 && n < 4) return whole;
   if (nkt >= 40) return units * 100 >= n * kCUs * 93;
-  return whole && n >= 2 && nkt >= (L.batch > 1 ? (n >= 3 ? 24 : 32) : (n >= 3 ? 32 : 36));
+  const bool sooner = L.batch > 1 || !L.use_corr;
+  return whole && n >= 2 && nkt >= (sooner ? (n >= 3 ? 24 : 32) : (n >= 3 ? 32 : 36));
 }
 
 void make_product_layout(int64_t batch, int64_t M, int64_t N, int64_t K, int P, bool corr,
