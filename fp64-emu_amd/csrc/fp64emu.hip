@@ -815,18 +815,13 @@ __device__ __forceinline__ void row_pass(const double* __restrict__ x, int64_t c
   }
 }
 
-// kGroup: few rows (not enough waves to fill the chip): a 256-thread group
-// per row, its wave w running sum 64 w + l alone (sixteen of its loads in
-// flight), the four waves' sums meeting in LDS before the same fold.  A
-// block of kWaves waves holds kWaves / 4 such groups, or kWaves rows (one
-// per wave) otherwise.
 // Short rows (at most kShortRow elements) in numbers that fill the chip: a
 // wave takes kShortRows rows, all of two rows' loads in flight, and folds
 // their 64 lane sums together: each of the first three tree steps sends half
 // of the lane's rows across and keeps the other half (the same pairs added as
 // one row's tree adds them; a + b and b + a are the same bits), so the eight
 // rows cost 10 exchanges instead of 48, and their logarithms are taken side by
-// side.  Whole calls, a wave a row / eight: 64 x 256^3 (32768 rows) 110 / 105
+// side.  Whole calls, a wave a row / eight: 64 x 256^3 (32768 rows) 116 / 111
 // us, 200 x 128^3 93 / 86, 100 x 200^3 157 / 148, 32 x 512^2 x 300 179 / 170;
 // even at 8192 rows (64 x 64^3) and slower at 512 elements (64 x 512^3 477 /
 // 482), whose loads alone fill the memory's queues.  Not for A's rows beside
@@ -904,6 +899,11 @@ __device__ __forceinline__ void size_short_rows(int64_t row0, const double* __re
   else row_stats_out(m[0], t[0], bits, &sftB[row - rowsA], &lgB[row - rowsA]);
 }
 
+// kGroup: few rows (not enough waves to fill the chip): a 256-thread group
+// per row, its wave w running sum 64 w + l alone (sixteen of its loads in
+// flight), the four waves' sums meeting in LDS before the same fold.  A
+// block of kWaves waves holds kWaves / 4 such groups, or kWaves rows (one
+// per wave) otherwise.
 template <bool kGroup, int kWaves>
 __device__ __forceinline__ void size_rows_body(int64_t bid, const double* __restrict__ A, int64_t rowsA,
                                                const double* __restrict__ B, int64_t rows, int64_t K,
@@ -3557,7 +3557,7 @@ fused_kernel(FusedArgs g) {
   };
   // A slot's first k-steps, no more than it has: every load takes the CU's
   // one vector memory path 16 cycles (redundant ones at the ends cost 64^3
-  // 14.2 us instead of 13.2, 64 x 256^3 104.8 instead of 100.6).
+  // 14.2 us instead of 13.2, 64 x 256^3 111.2 instead of 104.8).
   auto prefetch = [&](const int t) {
 #pragma unroll
     for (int d = 0; d < kD; ++d)

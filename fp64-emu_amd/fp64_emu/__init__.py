@@ -3,9 +3,10 @@
 Each operand is scaled by powers of two, per row of A and per column of B,
 to integers of at most 53 bits.  Their product is then known exactly
 through its remainders modulo a list of small pairwise-coprime moduli, and
-each remainder costs one INT8 MFMA GEMM of balanced residues.  A mixed-radix
-(Garner) recombination of those remainders, plus two int8 GEMMs of the
-rounding residue that correct the scaling's first-order error, gives the
+each remainder costs one INT8 MFMA GEMM of balanced residues.  The exact
+recombination of those remainders (by their Chinese remainder weights in the
+default plans, by mixed-radix Garner digits otherwise), plus two int8 GEMMs of
+the rounding residue that correct the scaling's first-order error, gives the
 float64 result.  How many moduli suffice is decided from K by the planner
 below, and a norm bound computed on the device narrows the integers until
 the product fits their range.  Integer inputs whose products are exact in

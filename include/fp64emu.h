@@ -3,7 +3,7 @@
  *
  * C = A @ B in float64 is recovered from INT8 products modulo up to 20
  * pairwise-coprime moduli (one CDNA4 INT8-MFMA GEMM each), a first-order
- * quantization correction (hi7 x q7 cross GEMMs) and balanced-Garner
+ * quantization correction (hi7 x q7 cross GEMMs) and an exact
  * reconstruction.  Every entry point enqueues asynchronously on `stream`
  * and allocates nothing: the caller passes a 256-byte aligned device
  * workspace of at least fp64emu_workspace_size() bytes (hipMalloc and the
